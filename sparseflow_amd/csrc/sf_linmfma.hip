@@ -586,6 +586,275 @@ __global__ __launch_bounds__(64 * kLbWaves, 2) void k_linear_bits_mfma(LinMfmaAr
                              lane);
 }
 
+// ---- wide tiles: x staged once for 384 output columns ---------------------
+//
+// k_linear_mfma's 128 x 128 tiles read (and convert) x once per 128 columns
+// and spend a step's time on staging: 32 MFMAs per wavefront between two
+// barriers.  Here a workgroup of 8 wavefronts computes 16 RT rows x 384
+// columns, each wavefront all rows of 48 columns (RT x 3 MFMA tiles, 6 RT
+// MFMAs a step): x is read, tested and converted once for all of them.  x
+// goes global -> registers (three steps ahead) -> bf16 in LDS (two steps
+// ahead, the conversion between the MFMAs), through four LDS buffers, so
+// that one barrier serves two steps; W's hi and lo tiles come by direct loads
+// into the other of two buffers and need no barrier, since a wavefront reads
+// only the columns it has loaded itself.  A second walk (x's lo part times
+// W hi) only where a workgroup saw an element that is not exact in bf16, as
+// in k_linear_mfma; same sums in the same order as there.
+// Bound by the matrix cores at the rate they hold under load: 50176 x 1536 ->
+// 384 runs in 121-127 us, 0.93-0.98 PFLOP/s counting both products (a plain
+// bf16 8192^3 product reaches 1.2 here); 191-212 us with k_linear_mfma.
+// With x staged one step ahead through two buffers and a barrier per step:
+// 125.7; all of a step's staging before its MFMAs, or half of it after them:
+// 131, 134.6.
+constexpr int kLwWaves = 8;
+constexpr int kLwCT = 3;                             // 16-column tiles per wavefront
+constexpr int kLwCols = 16 * kLwCT * kLwWaves;       // 384 columns per workgroup
+constexpr int kLwWBytes = kLwCols * kLmLda * 2;      // one part of a step's W tiles
+constexpr int kLwXBufs = 4;
+template <int RT> constexpr int lw_xbytes() { return 16 * RT * kLmLda * 2; }
+template <int RT> constexpr int lw_lds() { return 4 * kLwWBytes + kLwXBufs * lw_xbytes<RT>(); }
+
+typedef unsigned int lw_u32x4 __attribute__((ext_vector_type(4)));
+
+// 16 bytes per lane from the raw buffer rs at byte vo + so to LDS byte
+// address lds + 16 * lane.  In asm: the compiler would make every later LDS
+// read wait for every direct load in flight.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 in the clobber list
+__device__ __forceinline__ void lw_load_lds(lw_u32x4 rs, int vo, int so, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(vo), "s"(rs), "s"(so),
+               "s"(lds)
+               : "m0", "memory");
+}
+#pragma clang diagnostic pop
+
+__device__ __forceinline__ lw_u32x4 lw_rsrc(const void* p, uint32_t bytes) {
+  const uint64_t b = reinterpret_cast<uint64_t>(p);
+  return lw_u32x4{(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, bytes, 0x00020000u};
+}
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t lw_bf16x2(float v0, float v1) {  // round to nearest even, low half = v0
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{v0, v1}, bf16x2));
+}
+
+template <int RT>
+__global__ __launch_bounds__(64 * kLwWaves, 2) void k_linear_wide(LinMfmaArgs a) {
+  extern __shared__ __align__(16) char smem[];
+  constexpr int M = 16 * RT;
+  constexpr int NX = (M + 63) / 64;  // x loads per thread and step: 64 rows x 8 pieces of four elements each
+  constexpr int kXb = lw_xbytes<RT>();
+  char* const s_x = smem + 4 * kLwWBytes;  // after two buffers of W's hi and lo tiles
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ncb = (a.c_out + kLwCols - 1) / kLwCols;
+  const int bid = xcd_range_block((int)blockIdx.x, (int)gridDim.x);
+  const int64_t rb = bid / ncb;
+  const int64_t r0 = rb * M;
+  const int c0 = (int)(bid - rb * ncb) * kLwCols;
+  const int nsteps = a.kp / kLmK;
+  const float* __restrict__ X = static_cast<const float*>(a.x);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+
+  // x: thread t takes rows t / 8 + 64 j, elements 4 (t % 8) .. + 3 of the
+  // step.  Rows past m read the last one (their outputs are not stored).
+  const int xr = (int)threadIdx.x >> 3, xp = (int)threadIdx.x & 7;
+  f32x4 xv[NX];
+  auto load_piece = [&](int s, int j) {
+    const int kk = min(s * kLmK + 4 * xp, a.k - 4);
+    int64_t row = r0 + min(xr + 64 * j, M - 1);
+    row = row < a.m ? row : a.m - 1;
+    xv[j] = *reinterpret_cast<const f32x4*>(X + row * a.k + kk);
+  };
+  uint32_t inexact = 0u;  // some bit set: an element whose lo part is not zero
+  auto stage_piece = [&](int s, int j, auto lo_walk) {
+    constexpr bool LO = decltype(lo_walk)::value;
+    char* xb = s_x + (s % kLwXBufs) * kXb;
+    const bool in = s * kLmK + 4 * xp < a.k;  // k is a multiple of 4
+    {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = xv[j][e];
+        v[e] = in && fabsf(v[e]) >= a.cutoff ? v[e] : 0.f;  // the prescan's activity test
+      }
+      uint32_t h0 = lw_bf16x2(v[0], v[1]), h1 = lw_bf16x2(v[2], v[3]);
+      const float l0 = v[0] - __uint_as_float(h0 << 16), l1 = v[1] - __uint_as_float(h0 & 0xffff0000u);
+      const float l2 = v[2] - __uint_as_float(h1 << 16), l3 = v[3] - __uint_as_float(h1 & 0xffff0000u);
+      if constexpr (LO) {
+        h0 = lw_bf16x2(l0, l1);
+        h1 = lw_bf16x2(l2, l3);
+      } else {
+        inexact |= (__float_as_uint(l0) | __float_as_uint(l1) | __float_as_uint(l2) | __float_as_uint(l3)) & 0x7fffffffu;
+      }
+      const int r = xr + 64 * j;
+      if (64 * (j + 1) <= M || r < M)
+        *reinterpret_cast<uint2*>(xb + r * (2 * kLmLda) + 16 * lm_piece(r, xp >> 1) + 8 * (xp & 1)) = make_uint2(h0, h1);
+    }
+  };
+  // W: unit u (1 KB) of a part holds columns 16 u .. 16 u + 15 of the tile;
+  // LDS position q of a unit holds column q >> 2, stored piece q & 3
+  // (lm_piece is its own inverse).  Columns past c_out read column 0 (never
+  // stored).  Wavefront w loads units 3 w .. 3 w + 2: its own columns.
+  const lw_u32x4 rs_h = lw_rsrc(a.wh, (uint32_t)((int64_t)a.c_out * a.kp * 2));
+  const lw_u32x4 rs_l = lw_rsrc(a.wl, (uint32_t)((int64_t)a.c_out * a.kp * 2));
+  int wvo[kLwCT];
+#pragma unroll
+  for (int j = 0; j < kLwCT; ++j) {
+    const int r = lane >> 2;
+    const int col = c0 + 16 * (kLwCT * wave + j) + r;
+    wvo[j] = ((col < a.c_out ? col : 0) * a.kp + 8 * lm_piece(r, lane & 3)) * 2;
+  }
+  auto load_w = [&](int s, auto lo_walk) {
+    constexpr bool LO = decltype(lo_walk)::value;
+    const uint32_t b = lds0 + (uint32_t)((s & 1) * (2 * kLwWBytes));
+#pragma unroll
+    for (int j = 0; j < kLwCT; ++j) {
+      lw_load_lds(rs_h, wvo[j], s * (kLmK * 2), b + (uint32_t)(kLwCT * wave + j) * 1024u);
+      if constexpr (!LO) lw_load_lds(rs_l, wvo[j], s * (kLmK * 2), b + kLwWBytes + (uint32_t)(kLwCT * wave + j) * 1024u);
+    }
+  };
+
+  const int g = lane >> 4, li = lane & 15;
+  // MFMA operands W, x: register i of tile (rt, ct) is row 16 rt + li, column
+  // 16 ct + 4 g + i of the wavefront's 48: four consecutive columns a lane,
+  // stored without an exchange.
+  f32x4 acc[RT][kLwCT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int ct = 0; ct < kLwCT; ++ct) acc[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto walk = [&](auto lo_walk) {
+    constexpr bool LO = decltype(lo_walk)::value;
+    load_w(0, lo_walk);
+#pragma unroll
+    for (int j = 0; j < NX; ++j) load_piece(0, j);
+#pragma unroll
+    for (int j = 0; j < NX; ++j) stage_piece(0, j, lo_walk);
+    if (nsteps > 1) {
+#pragma unroll
+      for (int j = 0; j < NX; ++j) load_piece(1, j);
+#pragma unroll
+      for (int j = 0; j < NX; ++j) stage_piece(1, j, lo_walk);
+    }
+#pragma unroll
+    for (int j = 0; j < NX; ++j) load_piece(min(2, nsteps - 1), j);
+    ws_barrier();
+    for (int s = 0; s < nsteps; ++s) {
+      // This wavefront's W tiles of step s and its x of step s + 2, both
+      // requested a step ago, have landed (the x is used from here on, so
+      // that the compiler's own wait comes before the next direct loads).
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int j = 0; j < NX; ++j) asm volatile("" : "+v"(xv[j]));
+      if (s + 1 < nsteps) load_w(s + 1, lo_walk);
+      const bool more = s + 2 < nsteps;
+      const char* buf = smem + (s & 1) * (2 * kLwWBytes);
+      const char* xbuf = s_x + (s % kLwXBufs) * kXb;
+      bf16x8 bh[kLwCT], bl[kLwCT];
+#pragma unroll
+      for (int ct = 0; ct < kLwCT; ++ct) {
+        const int r = 16 * (kLwCT * wave + ct) + li;
+        const char* p = buf + r * (2 * kLmLda) + 16 * lm_piece(r, g);
+        bh[ct] = *reinterpret_cast<const bf16x8*>(p);
+        if constexpr (!LO) bl[ct] = *reinterpret_cast<const bf16x8*>(p + kLwWBytes);
+      }
+      auto read_x = [&](int rt) {
+        const int r = 16 * rt + li;
+        return *reinterpret_cast<const bf16x8*>(xbuf + r * (2 * kLmLda) + 16 * lm_piece(r, g));
+      };
+      bf16x8 ax = read_x(0);
+      // The step's row tiles, the next one's fragment requested ahead; the x
+      // of two steps on is converted and stored a piece at a time between them
+      // (and the one after it requested), so that it runs beside the MFMAs.
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        const bf16x8 an = read_x(rt + 1 < RT ? rt + 1 : rt);
+#pragma unroll
+        for (int ct = 0; ct < kLwCT; ++ct)
+          acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[ct], ax, acc[rt][ct], 0, 0, 0);
+        if constexpr (!LO) {
+#pragma unroll
+          for (int ct = 0; ct < kLwCT; ++ct)
+            acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl[ct], ax, acc[rt][ct], 0, 0, 0);
+        }
+        ax = an;
+#pragma unroll
+        for (int j = 0; j < NX; ++j)
+          if (rt == (j * RT) / NX) {
+            if (more) {
+              stage_piece(s + 2, j, lo_walk);
+              load_piece(min(s + 3, nsteps - 1), j);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+      }
+      // Steps 2 i and 2 i + 1 read two of the x buffers and write the other
+      // two: one barrier for both.
+      if (s & 1) ws_barrier();
+    }
+    ws_barrier();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
+  walk(std::false_type{});
+  if (__syncthreads_or(inexact != 0u ? 1 : 0)) walk(std::true_type{});
+
+  float* __restrict__ Y = static_cast<float*>(a.y);
+#pragma unroll
+  for (int ct = 0; ct < kLwCT; ++ct) {
+    const int col = c0 + 16 * (kLwCT * wave + ct) + 4 * g;
+    if (col >= a.c_out) continue;  // c_out is a multiple of 4
+    const f32x4 b = a.bias == nullptr ? f32x4{0.f, 0.f, 0.f, 0.f}
+                                      : f32x4{a.bias[col], a.bias[col + 1], a.bias[col + 2], a.bias[col + 3]};
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const int64_t row = r0 + 16 * rt + li;
+      if (row < a.m) *reinterpret_cast<f32x4*>(Y + row * a.c_out + col) = acc[rt][ct] + b;
+    }
+  }
+}
+
+// The number of 16-row tiles of a k_linear_wide workgroup, or 0 for
+// k_linear_mfma.  A step of a workgroup takes about 0.6 + 0.15 RT us however
+// many run, so: the fewest row tiles whose workgroups are all resident at
+// once, and 13 (all the accumulators that fit) past that, if the last round
+// of workgroups fills at least half of the CUs or so (tiles of whole rounds
+// >= 3/4).  us, k_linear_mfma -> wide, binary f32 x (x with a lo part gains
+// more: the second walk shares the staging):
+//   RT 4:  196 x 384 -> 384 16.2 -> 14.6;  1 x 2048 -> 1000 67.4 -> 51.7;
+//          12544 x 1536 -> 384 66.9 -> 50.1;  8192 x 512 -> 512 24.7 -> 22.3
+//   RT 8:  25088 x 384 -> 384 30.3 -> 26.5;  3136 x 768 -> 3072 55.9 -> 44.0
+//   RT 13: 50176 x 384 -> 384 50.7 -> 40.6;  20000 x 512 -> 1920 112 -> 86
+// Short K has no steps to hide the first loads and the stores behind (300 x
+// 128 -> 384 8.1 -> 8.4, 32000 x 128 -> 384 16.9 -> 17.9): k >= 192.  Columns
+// up to the next 384 are computed and dropped: up to half as many again are
+// paid back by the latency with 4 row tiles (16384 x 256 -> 256 14.9 -> 13.9),
+// not with more (16384 x 512 -> 512 31.7 -> 33.9, 40000 x 384 -> 256 31.6 ->
+// 34.0): an eighth there (32768 x 1024 -> 1024 175 -> 146).  75000 x 384 ->
+// 384 (1.4 rounds) stays at 64.3 with k_linear_mfma.
+int lw_row_tiles(const LinMfmaArgs& a, int in_dtype, int out_dtype) {
+  if (in_dtype != SF_F32 || out_dtype != SF_F32 || a.k < 192 || a.k % 4 != 0) return 0;
+  if (((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.y)) & 15) != 0) return 0;
+  if ((int64_t)a.c_out * a.kp * 2 >= (1ll << 31)) return 0;  // the buffer offsets' range
+  const int64_t cb = (a.c_out + kLwCols - 1) / kLwCols, cus = num_cus();
+  if (2 * cb * kLwCols <= 3 * (int64_t)a.c_out && (a.m + 63) / 64 * cb <= cus) return 4;
+  if (8 * cb * kLwCols > 9 * (int64_t)a.c_out) return 0;
+  if ((a.m + 127) / 128 * cb <= cus) return 8;
+  const int64_t tiles = (a.m + 207) / 208 * cb;
+  return 4 * tiles >= 3 * cus * ((tiles + cus - 1) / cus) ? 13 : 0;
+}
+
+template <int RT>
+int launch_lw_t(const LinMfmaArgs& a, hipStream_t stream) {
+  constexpr auto kern = k_linear_wide<RT>;
+  const int e = set_lds_limit_once<kern>(kMaxLdsBytes - 1024);  // (the block-wide OR takes a little)
+  if (e != (int)hipSuccess) return e;
+  const int64_t grid = ((a.m + 16 * RT - 1) / (16 * RT)) * ((a.c_out + kLwCols - 1) / kLwCols);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * kLwWaves), (size_t)lw_lds<RT>(), stream, a);
+  return (int)hipGetLastError();
+}
+
 template <typename TIn>
 int launch_lb_d(const LinMfmaArgs& a, const uint32_t* bits, const uint32_t* flags, int cwp, int out_dtype,
                 hipStream_t stream) {
@@ -636,6 +905,14 @@ int launch_linear_bits_mfma(const LinMfmaArgs& a, const uint32_t* bits, const ui
 
 int launch_linear_mfma(const LinMfmaArgs& a, int in_dtype, int out_dtype, hipStream_t stream) {
   timing_begin(K_LINEAR_MFMA, stream);
+  const int rt = lw_row_tiles(a, in_dtype, out_dtype);
+  if (rt != 0) {
+    const int rc = rt == 4   ? launch_lw_t<4>(a, stream)
+                   : rt == 8 ? launch_lw_t<8>(a, stream)
+                             : launch_lw_t<13>(a, stream);
+    timing_end(K_LINEAR_MFMA, stream);
+    return rc;
+  }
   const int rc = in_dtype == SF_F16    ? launch_lm_d<__half>(a, out_dtype, stream)
                  : in_dtype == SF_BF16 ? launch_lm_d<__hip_bfloat16>(a, out_dtype, stream)
                                        : launch_lm_d<float>(a, out_dtype, stream);

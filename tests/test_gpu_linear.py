@@ -239,3 +239,40 @@ def test_linear_random_shapes(case, kernel):
     assert ("linear_flat" if kernel == "walk" else "linear_mfma") in kernels, kernels
     ok, err, _ = close(y, olin.linear_ref(x, w, b), **FP32_TOL)
     assert ok, f"max abs err {err}"
+
+
+# The 384-column kernel: tiles of 64, 128 and 208 rows (by how many fill 256
+# CUs), rows and columns on both sides of a tile's end, k with and without a
+# remainder of 32, one K step past an even number of steps, x of one bit and of
+# full precision; k = 194 (not whole pieces of four), k = 188 (too short) and
+# an x that starts 4 bytes past 16 take the other kernel.
+WIDE_CASES = [(1, 192, 384), (64, 196, 260), (65, 384, 388), (16384, 224, 384), (16385, 224, 768), (32768, 192, 384),
+              (32769, 256, 384), (53249, 192, 384), (208 * 256, 192, 1536), (70, 194, 384), (70, 188, 384)]
+
+
+@pytest.mark.parametrize("case", WIDE_CASES)
+@pytest.mark.parametrize("form", ["binary", "values", "infinite"])
+def test_mfma_wide_tiles(case, form):
+    m, k, co = case
+    announce(f"linear wide tiles {case} {form}")
+    g = torch.Generator(device=DEV).manual_seed(m + k)
+    x = (torch.rand(m, k, generator=g, device=DEV) < 0.2).float()
+    if form != "binary":
+        x = x * torch.randn(m, k, generator=g, device=DEV)
+    if form == "infinite":  # a row of its own: inf there, the others untouched
+        x[m // 2, k - 1] = float("inf")
+    w = _w(co, k, seed=co).to(DEV)
+    b = (torch.randn(co, generator=torch.Generator().manual_seed(34)) * 0.1).to(DEV)
+    y, kernels = _run(x, w, b, kernel="mfma", threshold=1e-6)
+    assert set(kernels) == {"linear_mfma"}, kernels
+    off = torch.empty(m * k + 1, device=DEV)[1:].view(m, k).copy_(x)
+    y2, _ = _run(off, w, b, kernel="mfma", threshold=1e-6)
+    assert torch.equal(torch.nan_to_num(y), torch.nan_to_num(y2))  # the same sums in the same order
+    keep = torch.arange(m, device=DEV) != m // 2 if form == "infinite" else slice(None)
+    ref = torch.where(x.abs() >= 1e-6, x, 0.0)[keep].double() @ w.double().t() + b.double()
+    # W's hi + lo halves carry 16 bits: 2^-16 of sum |x| |w| at most, and the
+    # f32 sums add k roundings of the same magnitude at 2^-24.
+    bound = (2.0 ** -16 + k * 2.0 ** -24) * (x[keep].abs().double() @ w.abs().double().t()) + 1e-6
+    assert bool(((y[keep].double() - ref).abs() <= bound).all())
+    if form == "infinite":
+        assert not bool(torch.isfinite(y[m // 2]).any())
