@@ -639,13 +639,15 @@ __device__ __forceinline__ uint32_t lw_bf16x2(float v0, float v1) {  // round to
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{v0, v1}, bf16x2));
 }
 
-template <int RT>
+template <typename TIn, typename TOut, int RT, bool VEC>
 __global__ __launch_bounds__(64 * kLwWaves, 2) void k_linear_wide(LinMfmaArgs a) {
   extern __shared__ __align__(16) char smem[];
   constexpr int M = 16 * RT;
   constexpr int NX = (M + 63) / 64;  // x loads per thread and step: 64 rows x 8 pieces of four elements each
   constexpr int kXb = lw_xbytes<RT>();
   char* const s_x = smem + 4 * kLwWBytes;  // after two buffers of W's hi and lo tiles
+  // VEC: k a multiple of four, x on whole pieces; otherwise rows start anywhere.
+  struct __attribute__((packed, aligned((VEC ? 4 : 1) * sizeof(TIn)))) X4 { TIn e[4]; };
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ncb = (a.c_out + kLwCols - 1) / kLwCols;
@@ -654,29 +656,35 @@ __global__ __launch_bounds__(64 * kLwWaves, 2) void k_linear_wide(LinMfmaArgs a)
   const int64_t r0 = rb * M;
   const int c0 = (int)(bid - rb * ncb) * kLwCols;
   const int nsteps = a.kp / kLmK;
-  const float* __restrict__ X = static_cast<const float*>(a.x);
+  const TIn* __restrict__ X = static_cast<const TIn*>(a.x);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
 
   // x: thread t takes rows t / 8 + 64 j, elements 4 (t % 8) .. + 3 of the
   // step.  Rows past m read the last one (their outputs are not stored).
   const int xr = (int)threadIdx.x >> 3, xp = (int)threadIdx.x & 7;
-  f32x4 xv[NX];
+  X4 xv[NX];
   auto load_piece = [&](int s, int j) {
-    const int kk = min(s * kLmK + 4 * xp, a.k - 4);
+    const int kk = s * kLmK + 4 * xp;
     int64_t row = r0 + min(xr + 64 * j, M - 1);
     row = row < a.m ? row : a.m - 1;
-    xv[j] = *reinterpret_cast<const f32x4*>(X + row * a.k + kk);
+    const TIn* p = X + row * a.k;
+    if (VEC || s * kLmK + kLmK <= a.k) {
+      xv[j] = *reinterpret_cast<const X4*>(p + (VEC ? min(kk, a.k - 4) : kk));  // (not staged where kk >= k)
+    } else {  // the last step of a ragged k: element by element, 0 past the row's end
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xv[j].e[e] = kk + e < a.k ? p[kk + e] : from_f32<TIn>(0.f);
+    }
   };
   uint32_t inexact = 0u;  // some bit set: an element whose lo part is not zero
   auto stage_piece = [&](int s, int j, auto lo_walk) {
     constexpr bool LO = decltype(lo_walk)::value;
     char* xb = s_x + (s % kLwXBufs) * kXb;
-    const bool in = s * kLmK + 4 * xp < a.k;  // k is a multiple of 4
+    const bool in = !VEC || s * kLmK + 4 * xp < a.k;
     {
       float v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v[e] = xv[j][e];
+        v[e] = to_f32<TIn>(xv[j].e[e]);
         v[e] = in && fabsf(v[e]) >= a.cutoff ? v[e] : 0.f;  // the prescan's activity test
       }
       uint32_t h0 = lw_bf16x2(v[0], v[1]), h1 = lw_bf16x2(v[2], v[3]);
@@ -747,7 +755,12 @@ __global__ __launch_bounds__(64 * kLwWaves, 2) void k_linear_wide(LinMfmaArgs a)
       // that the compiler's own wait comes before the next direct loads).
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-      for (int j = 0; j < NX; ++j) asm volatile("" : "+v"(xv[j]));
+      for (int j = 0; j < NX; ++j) {
+        typedef unsigned int u32xn __attribute__((ext_vector_type(sizeof(X4) / 4)));
+        u32xn q = __builtin_bit_cast(u32xn, xv[j]);
+        asm volatile("" : "+v"(q));
+        xv[j] = __builtin_bit_cast(X4, q);
+      }
       if (s + 1 < nsteps) load_w(s + 1, lo_walk);
       const bool more = s + 2 < nsteps;
       const char* buf = smem + (s & 1) * (2 * kLwWBytes);
@@ -800,7 +813,7 @@ __global__ __launch_bounds__(64 * kLwWaves, 2) void k_linear_wide(LinMfmaArgs a)
   walk(std::false_type{});
   if (__syncthreads_or(inexact != 0u ? 1 : 0)) walk(std::true_type{});
 
-  float* __restrict__ Y = static_cast<float*>(a.y);
+  TOut* __restrict__ Y = static_cast<TOut*>(a.y);
 #pragma unroll
   for (int ct = 0; ct < kLwCT; ++ct) {
     const int col = c0 + 16 * (kLwCT * wave + ct) + 4 * g;
@@ -810,18 +823,43 @@ __global__ __launch_bounds__(64 * kLwWaves, 2) void k_linear_wide(LinMfmaArgs a)
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       const int64_t row = r0 + 16 * rt + li;
-      if (row < a.m) *reinterpret_cast<f32x4*>(Y + row * a.c_out + col) = acc[rt][ct] + b;
+      const f32x4 v = acc[rt][ct] + b;
+      if (row < a.m) store4<TOut>(Y + row * a.c_out + col, v[0], v[1], v[2], v[3]);
     }
   }
 }
 
+template <typename TIn>
+bool lm_vec(const LinMfmaArgs& a) {  // k_linear_mfma's 16-byte loads
+  return sizeof(TIn) == 4 && a.k % 16 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0;
+}
+
 // The number of 16-row tiles of a k_linear_wide workgroup, or 0 for
-// k_linear_mfma.  A step of a workgroup takes about 0.6 + 0.15 RT us however
-// many run, so: the fewest row tiles whose workgroups are all resident at
-// once, and 13 (all the accumulators that fit) past that, if the last round
-// of workgroups fills at least half of the CUs or so (tiles of whole rounds
-// >= 3/4).  us, k_linear_mfma -> wide, binary f32 x (x with a lo part gains
-// more: the second walk shares the staging):
+// k_linear_mfma.
+//
+// A K step of a workgroup takes about 0.6 + 0.15 RT us however many run, one
+// workgroup a CU: of 4, 8 and 13 row tiles (all the accumulators that fit)
+// the one whose rounds of workgroups take least.
+//
+// 16-bit x and f32 x with a k that is no multiple of 16 or a start off 16
+// bytes, where k_linear_mfma loads and converts single elements: from 128
+// columns and k 48 on, but past one round of workgroups only with a k of
+// whole pieces of four or at least 160 (a ragged k's last step loads single
+// elements here too); one round of 4 row tiles, or of a k from 192 on, pays
+// at any width.  us, k_linear_mfma -> wide:
+//   f16 (bf16 the same)  50176 x 384 -> 384 135 -> 41.7;  8192 x 512 -> 2048
+//   146 -> 49.9;  1000 x 128 -> 128 14.5 -> 7.9;  100000 x 128 -> 128 43.1 ->
+//   37.4;  50000 x 48 -> 192 19.3 -> 16.2;  50000 x 386 -> 384 104 -> 46.6;
+//   701 x 1790 -> 100 112 -> 48.4;  but 50000 x 64 -> 64 13.6 -> 14.5, 100000
+//   x 129 -> 128 35.8 -> 43.6
+//   f32  50176 x 1535 -> 384 479 -> 148;  1000 x 383 -> 384 26.7 -> 15.4;
+//   300 x 50 -> 128 7.6 -> 7.2;  30000 x 161 -> 640 53.7 -> 38.2;  200 x 1001
+//   -> 12 62.2 -> 26.6;  3000 x 99 -> 100 10.9 -> 8.0;  30000 x 200 -> 4 16.6 ->
+//   13.1;  but 65536 x 129 -> 512 65.2 -> 67.4, 100000 x 129 -> 128 37.3 -> 46.7,
+//   30000 x 99 -> 100 12.7 -> 13.8
+//
+// Other f32 x, binary (x with a lo part gains more: the second walk shares the
+// staging):
 //   RT 4:  196 x 384 -> 384 16.2 -> 14.6;  1 x 2048 -> 1000 67.4 -> 51.7;
 //          12544 x 1536 -> 384 66.9 -> 50.1;  8192 x 512 -> 512 24.7 -> 22.3
 //   RT 8:  25088 x 384 -> 384 30.3 -> 26.5;  3136 x 768 -> 3072 55.9 -> 44.0
@@ -829,30 +867,57 @@ __global__ __launch_bounds__(64 * kLwWaves, 2) void k_linear_wide(LinMfmaArgs a)
 // Short K has no steps to hide the first loads and the stores behind (300 x
 // 128 -> 384 8.1 -> 8.4, 32000 x 128 -> 384 16.9 -> 17.9): k >= 192.  Columns
 // up to the next 384 are computed and dropped: up to half as many again are
-// paid back by the latency with 4 row tiles (16384 x 256 -> 256 14.9 -> 13.9),
-// not with more (16384 x 512 -> 512 31.7 -> 33.9, 40000 x 384 -> 256 31.6 ->
-// 34.0): an eighth there (32768 x 1024 -> 1024 175 -> 146).  75000 x 384 ->
-// 384 (1.4 rounds) stays at 64.3 with k_linear_mfma.
-int lw_row_tiles(const LinMfmaArgs& a, int in_dtype, int out_dtype) {
-  if (in_dtype != SF_F32 || out_dtype != SF_F32 || a.k < 192 || a.k % 4 != 0) return 0;
-  if (((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.y)) & 15) != 0) return 0;
+// paid back by the latency in one round of 4 row tiles (16384 x 256 -> 256
+// 14.9 -> 13.9), not with more (16384 x 512 -> 512 31.7 -> 33.9, 40000 x 384
+// -> 256 31.6 -> 34.0): an eighth there (32768 x 1024 -> 1024 175 -> 146).
+// Past one round, the rounds at least three quarters full (100352 x 384 ->
+// 384, 0.94: 122 -> 87; 75000 x 384 -> 384, 0.71: 64.3 with k_linear_mfma).
+template <typename TIn>
+int lw_row_tiles(const LinMfmaArgs& a) {
   if ((int64_t)a.c_out * a.kp * 2 >= (1ll << 31)) return 0;  // the buffer offsets' range
   const int64_t cb = (a.c_out + kLwCols - 1) / kLwCols, cus = num_cus();
-  if (2 * cb * kLwCols <= 3 * (int64_t)a.c_out && (a.m + 63) / 64 * cb <= cus) return 4;
+  int rt = 0;
+  int64_t best = 0, tiles = 0;
+  for (const int r : {4, 8, 13}) {
+    const int64_t t = (a.m + 16 * r - 1) / (16 * r) * cb, cost = (t + cus - 1) / cus * (4 + r);
+    if (rt == 0 || cost < best) {
+      rt = r;
+      best = cost;
+      tiles = t;
+    }
+  }
+  if (!lm_vec<TIn>(a)) {
+    if (tiles <= cus) return (a.c_out >= 128 && a.k >= 48) || rt == 4 || a.k >= 192 ? rt : 0;
+    return a.c_out >= 128 && a.k >= 48 && (a.k % 4 == 0 || a.k >= 160) ? rt : 0;
+  }
+  if (a.k < 192) return 0;
+  if (rt == 4 && tiles <= cus) return 2 * cb * kLwCols <= 3 * (int64_t)a.c_out ? rt : 0;
   if (8 * cb * kLwCols > 9 * (int64_t)a.c_out) return 0;
-  if ((a.m + 127) / 128 * cb <= cus) return 8;
-  const int64_t tiles = (a.m + 207) / 208 * cb;
-  return 4 * tiles >= 3 * cus * ((tiles + cus - 1) / cus) ? 13 : 0;
+  return tiles <= cus || 4 * tiles >= 3 * cus * ((tiles + cus - 1) / cus) ? rt : 0;
 }
 
-template <int RT>
+template <typename TIn, typename TOut, int RT, bool VEC>
 int launch_lw_t(const LinMfmaArgs& a, hipStream_t stream) {
-  constexpr auto kern = k_linear_wide<RT>;
+  constexpr auto kern = k_linear_wide<TIn, TOut, RT, VEC>;
   const int e = set_lds_limit_once<kern>(kMaxLdsBytes - 1024);  // (the block-wide OR takes a little)
   if (e != (int)hipSuccess) return e;
   const int64_t grid = ((a.m + 16 * RT - 1) / (16 * RT)) * ((a.c_out + kLwCols - 1) / kLwCols);
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * kLwWaves), (size_t)lw_lds<RT>(), stream, a);
   return (int)hipGetLastError();
+}
+
+template <typename TIn, typename TOut, bool VEC>
+int launch_lw_v(const LinMfmaArgs& a, int rt, hipStream_t stream) {
+  return rt == 4   ? launch_lw_t<TIn, TOut, 4, VEC>(a, stream)
+         : rt == 8 ? launch_lw_t<TIn, TOut, 8, VEC>(a, stream)
+                   : launch_lw_t<TIn, TOut, 13, VEC>(a, stream);
+}
+
+template <typename TIn, typename TOut>
+int launch_lw(const LinMfmaArgs& a, int rt, hipStream_t stream) {
+  return a.k % 4 == 0 && reinterpret_cast<uintptr_t>(a.x) % (4 * sizeof(TIn)) == 0
+             ? launch_lw_v<TIn, TOut, true>(a, rt, stream)
+             : launch_lw_v<TIn, TOut, false>(a, rt, stream);
 }
 
 template <typename TIn>
@@ -871,11 +936,12 @@ int launch_lb_d(const LinMfmaArgs& a, const uint32_t* bits, const uint32_t* flag
 
 template <typename TIn>
 int launch_lm_d(const LinMfmaArgs& a, int out_dtype, hipStream_t stream) {
+  const int rt = lw_row_tiles<TIn>(a);
+  if (rt != 0) return out_dtype == SF_F32 ? launch_lw<TIn, float>(a, rt, stream) : launch_lw<TIn, TIn>(a, rt, stream);
   const int64_t rbs = (a.m + kLmRows - 1) / kLmRows;
   const int64_t grid = rbs * ((a.c_out + kLmCols - 1) / kLmCols);
   if (grid == 0) return (int)hipSuccess;
-  const bool vec = sizeof(TIn) == 4 && a.k % 16 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0;
-  if (vec) {
+  if (lm_vec<TIn>(a)) {
     if (out_dtype == SF_F32)
       hipLaunchKernelGGL((k_linear_mfma<TIn, float, true>), dim3((unsigned)grid), dim3(256), 0, stream, a);
     else
@@ -905,14 +971,6 @@ int launch_linear_bits_mfma(const LinMfmaArgs& a, const uint32_t* bits, const ui
 
 int launch_linear_mfma(const LinMfmaArgs& a, int in_dtype, int out_dtype, hipStream_t stream) {
   timing_begin(K_LINEAR_MFMA, stream);
-  const int rt = lw_row_tiles(a, in_dtype, out_dtype);
-  if (rt != 0) {
-    const int rc = rt == 4   ? launch_lw_t<4>(a, stream)
-                   : rt == 8 ? launch_lw_t<8>(a, stream)
-                             : launch_lw_t<13>(a, stream);
-    timing_end(K_LINEAR_MFMA, stream);
-    return rc;
-  }
   const int rc = in_dtype == SF_F16    ? launch_lm_d<__half>(a, out_dtype, stream)
                  : in_dtype == SF_BF16 ? launch_lm_d<__hip_bfloat16>(a, out_dtype, stream)
                                        : launch_lm_d<float>(a, out_dtype, stream);

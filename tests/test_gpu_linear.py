@@ -243,36 +243,48 @@ def test_linear_random_shapes(case, kernel):
 
 # The 384-column kernel: tiles of 64, 128 and 208 rows (by how many fill 256
 # CUs), rows and columns on both sides of a tile's end, k with and without a
-# remainder of 32, one K step past an even number of steps, x of one bit and of
-# full precision; k = 194 (not whole pieces of four), k = 188 (too short) and
-# an x that starts 4 bytes past 16 take the other kernel.
+# remainder of 32 and of 4, an odd number of K steps, x of one bit and of full
+# precision, x that starts one element past 16 bytes.  f32 x with k = 176 takes
+# it only from such a start, 53249 rows of k = 50 never do.
 WIDE_CASES = [(1, 192, 384), (64, 196, 260), (65, 384, 388), (16384, 224, 384), (16385, 224, 768), (32768, 192, 384),
-              (32769, 256, 384), (53249, 192, 384), (208 * 256, 192, 1536), (70, 194, 384), (70, 188, 384)]
+              (32769, 256, 384), (53249, 193, 384), (208 * 256, 192, 1536), (70, 194, 384), (70, 176, 384),
+              (300, 48, 128), (300, 3, 4), (300, 44, 124), (209, 51, 132), (53249, 50, 128), (9, 415, 1000)]
 
 
-@pytest.mark.parametrize("case", WIDE_CASES)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("form", ["binary", "values", "infinite"])
-def test_mfma_wide_tiles(case, form):
+@pytest.mark.parametrize("case", WIDE_CASES)
+def test_mfma_wide_tiles(case, form, dtype):
     m, k, co = case
-    announce(f"linear wide tiles {case} {form}")
+    announce(f"linear wide tiles {case} {form} {dtype}")
     g = torch.Generator(device=DEV).manual_seed(m + k)
     x = (torch.rand(m, k, generator=g, device=DEV) < 0.2).float()
     if form != "binary":
         x = x * torch.randn(m, k, generator=g, device=DEV)
-    if form == "infinite":  # a row of its own: inf there, the others untouched
+    x = x.to(dtype)
+    if form == "infinite":  # a row of its own: not finite there, the others untouched
         x[m // 2, k - 1] = float("inf")
     w = _w(co, k, seed=co).to(DEV)
     b = (torch.randn(co, generator=torch.Generator().manual_seed(34)) * 0.1).to(DEV)
-    y, kernels = _run(x, w, b, kernel="mfma", threshold=1e-6)
+    y, kernels = _run(x, w, b, kernel="mfma", threshold=1e-6, output_dtype=torch.float32)
     assert set(kernels) == {"linear_mfma"}, kernels
-    off = torch.empty(m * k + 1, device=DEV)[1:].view(m, k).copy_(x)
-    y2, _ = _run(off, w, b, kernel="mfma", threshold=1e-6)
+    off = torch.empty(m * k + 1, device=DEV, dtype=dtype)[1:].view(m, k).copy_(x)
+    y2, _ = _run(off, w, b, kernel="mfma", threshold=1e-6, output_dtype=torch.float32)
     assert torch.equal(torch.nan_to_num(y), torch.nan_to_num(y2))  # the same sums in the same order
+    ya, _ = _run(x, w, b, threshold=1e-6)  # x's own type, the default's choice of kernel
     keep = torch.arange(m, device=DEV) != m // 2 if form == "infinite" else slice(None)
-    ref = torch.where(x.abs() >= 1e-6, x, 0.0)[keep].double() @ w.double().t() + b.double()
-    # W's hi + lo halves carry 16 bits: 2^-16 of sum |x| |w| at most, and the
-    # f32 sums add k roundings of the same magnitude at 2^-24.
-    bound = (2.0 ** -16 + k * 2.0 ** -24) * (x[keep].abs().double() @ w.abs().double().t()) + 1e-6
+    # Below k = 32 the default is the f32 walk; with lo parts the bitmap kernel
+    # adds them step by step, the direct ones in a second walk.
+    if form == "binary" and k >= 32:
+        assert torch.equal(ya[keep], y[keep].to(dtype))
+    xd = torch.where(x.abs().float() >= 1e-6, x.float(), 0.0)[keep].double()
+    ref = xd @ w.double().t() + b.double()
+    # A bf16 rounds to 8 bits (2^-8 at most), hi + lo to 2^-16: what W's halves
+    # lose, what x's lose (nothing when binary) and x lo * W lo, left out, are
+    # 2^-16 of sum |x| |w| each; the f32 sums (two per element) add 2^-24 each.
+    bound = ((1 if form == "binary" else 3) * 2.0 ** -16 + 3 * k * 2.0 ** -24) * (xd.abs() @ w.abs().double().t()) + 1e-6
     assert bool(((y[keep].double() - ref).abs() <= bound).all())
+    half = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    assert bool(((ya[keep].double() - ref).abs() <= bound + half * (ref.abs() + bound)).all())
     if form == "infinite":
         assert not bool(torch.isfinite(y[m // 2]).any())
