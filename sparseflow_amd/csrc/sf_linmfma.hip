@@ -352,7 +352,7 @@ __device__ __forceinline__ void lb_load_w(uint16_t* __restrict__ sh, uint16_t* _
     const int col = c0 + r < c_out ? c0 + r : 0;
     const uint16_t* src = (u < 8 ? wh : wl) + (int64_t)col * kp + 32 * s + 8 * p;
     uint16_t* dst = (u < 8 ? sh : sl) + (u & 7) * 512;  // 1 KB = 512 bf16
-    __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)dst, 16, 0, 0);
+    lds_dma16(src, dst);
   }
 }
 constexpr int kLbLoads = 16 / kLbWaves + 1;  // direct loads per wavefront and step (W blocks, words)
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(64 * kLbWaves, 2) void k_linear_bits_mfma(LinMfmaAr
     const int q = 64 * wave + lane;
     const int64_t row = r0 + 128 * (q >> 7) + 16 * (q & 7) + ((q >> 3) & 15);
     const uint32_t* src = bits + (row < a.m ? row : 0) * (int64_t)cwp + t;
-    __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)&s_words[b][64 * wave], 4, 0, 0);
+    lds_dma4(src, &s_words[b][64 * wave]);
   };
   auto bfrags = [&](int b, bf16x8 (&bh)[4], bf16x8 (&bl)[4]) {
 #pragma unroll

@@ -83,7 +83,7 @@ __device__ __forceinline__ void load_chunk_px3(char* buf, const float* __restric
       const int col = co0 + 4 * s;
       const float* src =
           (q < L::pieces && r < kPx3Rows && row < krows && col < c_out) ? wt + (int64_t)row * c_out + col : wt;
-      __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)(buf + u * 1024), 16, 0, 0);
+      lds_dma16(src, buf + u * 1024);
     }
   }
 }
@@ -119,6 +119,26 @@ __device__ __forceinline__ void px3_add_row_at(float (&acc)[CO], const char* row
     acc[4 * s + 1] = fmaf(xv, v.y, acc[4 * s + 1]);
     acc[4 * s + 2] = fmaf(xv, v.z, acc[4 * s + 2]);
     acc[4 * s + 3] = fmaf(xv, v.w, acc[4 * s + 3]);
+  }
+}
+
+// Add CW of a 64-channel row's channels (from rowp on, immediate offsets),
+// times xv.  Fewer than 64 leave registers for all of a spike's reads.
+template <int CW>
+__device__ __forceinline__ void px3_add_pieces(float (&acc)[CW], const char* rowp, float xv) {
+  if constexpr (CW == 64) {
+    px3_add_row_at<64>(acc, rowp, 0, xv);
+  } else {
+    float4 v[CW / 4];
+#pragma unroll
+    for (int s = 0; s < CW / 4; ++s) v[s] = reinterpret_cast<const float4*>(rowp)[s];
+#pragma unroll
+    for (int s = 0; s < CW / 4; ++s) {
+      acc[4 * s] = fmaf(xv, v[s].x, acc[4 * s]);
+      acc[4 * s + 1] = fmaf(xv, v[s].y, acc[4 * s + 1]);
+      acc[4 * s + 2] = fmaf(xv, v[s].z, acc[4 * s + 2]);
+      acc[4 * s + 3] = fmaf(xv, v[s].w, acc[4 * s + 3]);
+    }
   }
 }
 
@@ -304,7 +324,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3(ConvArgs a, const 
   if (resident) {
     for (int c = 0; c < nchunks; ++c)
       load_chunk_px3<CO>(smem + c * LY::chunk_bytes, wt, c, krows, a.c_out, co0, wave, lane0);
-    __builtin_amdgcn_s_waitcnt(0);
+    lds_dma_wait();
     __syncthreads();
   }
   // First-chunk bitmap words of the next tile (or the next step) are always
@@ -377,7 +397,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3(ConvArgs a, const 
         int ll = lane;
         asm volatile("" : "+v"(ll));
         load_chunk_px3<CO>(smem, wt, 0, krows, a.c_out, co0, wave, ll);
-        __builtin_amdgcn_s_waitcnt(0);
+        lds_dma_wait();
         __syncthreads();
       }
       for (int c = 0; c < nchunks; ++c) {
@@ -429,7 +449,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3(ConvArgs a, const 
           }
         }
         if (!resident) {
-          __builtin_amdgcn_s_waitcnt(0);
+          lds_dma_wait();
           __syncthreads();
         }
       }
@@ -478,6 +498,18 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3(ConvArgs a, const 
 // (chunk, tap, ci) order, as there.
 // ---------------------------------------------------------------------------
 
+// Up to this many tiles per workgroup, four wavefronts walk a tile, 16 output
+// channels each (the same sums in the same order); wavefronts up to
+// kRowsWaves that have no tile load weights.  A tile's walk and, with few
+// wavefronts, the chunk loads are serial chains that nothing else on the CU
+// hides: 74 x 509 x 8 x 7 -> 48 (clustered spikes, 65 tiles) took 187 us, 141
+// of them loading with one wavefront per CU; loads by 16 wavefronts 69 us,
+// walked by four 48 us.  98 x 451 x 19 x 18 -> 40 157 -> 124 -> 84, 101 x 144 x
+// 15 x 15 -> 52 46.8 -> 31 -> 23, 10 x 191 x 8 x 8 -> 60 70 -> 27 -> 22.  Five to
+// eight tiles walked by two wavefronts each gain nothing (512 x 512 x 14 x 14 ->
+// 512 stride 2 152.6 / 152.1 us, 158 x 319 x 44 x 44 -> 52 120 / 115).
+constexpr int kPx3sSplitTiles = 4;
+
 // Direct-to-LDS loads of chunk c by the nw wavefronts of the workgroup.
 __device__ __forceinline__ void load_chunk_px3_nw(char* buf, const float* __restrict__ wt, int c, int krows,
                                                   int c_out, int co0, int wave, int nw, int lane) {
@@ -489,7 +521,7 @@ __device__ __forceinline__ void load_chunk_px3_nw(char* buf, const float* __rest
     const int row = c * kPx3Rows + r;
     const int col = co0 + 4 * q;
     const float* src = (q < L::pieces && r < kPx3Rows && row < krows && col < c_out) ? wt + (int64_t)row * c_out + col : wt;
-    __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)(buf + u * 1024), 16, 0, 0);
+    lds_dma16(src, buf + u * 1024);
   }
 }
 
@@ -497,17 +529,22 @@ __device__ __forceinline__ void load_chunk_px3_nw(char* buf, const float* __rest
 // kDenseLaneSpikes or more spikes in the first chunk is appended to its
 // group's queue and neither walked nor stored here: the matrix-core kernel
 // launched next computes it (sf_dense_mfma.hip).
-template <typename TIn, typename TOut>
+template <typename TIn, typename TOut, int CW>
 __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const uint32_t* __restrict__ bits,
                                                                const uint32_t* __restrict__ flags,
                                                                const TIn* __restrict__ x, const float* __restrict__ wt,
                                                                const float* __restrict__ bias_p, TOut* __restrict__ y,
-                                                               int groups, int nchunks, DenseQueue* __restrict__ dq) {
+                                                               int groups, int nchunks, int nt,
+                                                               DenseQueue* __restrict__ dq) {
   typedef Px3Layout<64> LY;
+  constexpr int SPLIT = 64 / CW;
   extern __shared__ __align__(16) char smem[];
   __shared__ float s_seed[64];
-  const int nw = __builtin_amdgcn_readfirstlane((int)(blockDim.x >> 6));
+  __shared__ uint32_t s_queued[kRowsWaves];  // per tile: on the dense queue
+  constexpr int nw = kRowsWaves;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = SPLIT == 1 ? wave : wave / SPLIT;  // of the workgroup's nt; past them: a wavefront that only loads
+  const int part = SPLIT == 1 ? 0 : wave % SPLIT;     // its channels: CW part ..
   const int blk = groups >= 8 ? xcd_local_block((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
   const int grp = blk % groups;
   const int co0 = grp * 64;
@@ -522,15 +559,15 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const
     const int co = co0 + (int)threadIdx.x;
     s_seed[threadIdx.x] = (bias_p != nullptr && co < a.c_out) ? bias_p[co] : 0.f;
   }
-  for (int pass = blk / groups; pass * nw < total; pass += nblk) {
+  for (int pass = blk / groups; pass * nt < total; pass += nblk) {
     // The lane index is formed anew in each pass (in asm, which the
     // optimiser cannot hoist): kept live across the loop it was spilled, and
     // its reload waited for the previous pass's stores.
     int lane;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
-    const int t = pass * nw + wave;
+    const int t = pass * nt + tile;
     const int g = t * 64 + lane;
-    const bool mine = g < total_px;
+    const bool mine = tile < nt && g < total_px;
     const int gc = mine ? g : total_px - 1;  // lanes past the end form valid addresses
     const int sample = gc / hwo;
     const int q = gc - sample * hwo;
@@ -543,7 +580,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const
     constexpr uint32_t B = (uint32_t)sizeof(TOut);
     const uint32_t yrange = (uint32_t)total_px * (uint32_t)a.c_out * B;
     uint32_t ybase =
-        mine ? (((uint32_t)sample * (uint32_t)a.c_out + (uint32_t)co0) * (uint32_t)hwo + (uint32_t)q) * B : yrange;
+        mine ? (((uint32_t)sample * (uint32_t)a.c_out + (uint32_t)(co0 + CW * part)) * (uint32_t)hwo + (uint32_t)q) * B : yrange;
     // This pass's first words, in flight during the first chunk's load.
     uint32_t wn[9];
     px3_load_words_at(wn, rs_bits, fbase, a, ih0, iw0, 0);
@@ -554,11 +591,13 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const
     // queued for the matrix cores instead of walked (its lanes then store
     // nothing here).
     bool walk = mine;
+    bool dense = false;
     if (dq != nullptr && !value) {
       uint32_t cnt = 0u;
 #pragma unroll
       for (int tp = 0; tp < 9; ++tp) cnt += (uint32_t)__popc(wn[tp]);
-      if (__ballot(mine && cnt >= (uint32_t)kDenseLaneSpikes) != 0ull) {
+      dense = __ballot(mine && cnt >= (uint32_t)kDenseLaneSpikes) != 0ull;
+      if (dense && part == 0) {
         uint32_t slot = 0u;
         if (lane == 0) slot = atomicAdd(&dq->count[grp], 1u);
         slot = __builtin_amdgcn_readfirstlane(slot);
@@ -567,6 +606,11 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const
             dq->start[grp][slot] = (uint32_t)t * 64u;
             dq->npx[grp][slot] = 64;  // the last tile's pixels past the end are not stored
           }
+        }
+        // The tile's other wavefronts read this behind the barrier; the next
+        // pass writes it behind this one's chunk barriers.
+        if (SPLIT > 1 && lane == 0) s_queued[tile] = slot < (uint32_t)kDenseQueueCap ? 1u : 0u;
+        if (SPLIT == 1 && slot < (uint32_t)kDenseQueueCap) {
           walk = false;
           ybase = yrange;
         }
@@ -578,10 +622,14 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const
       asm volatile("" : "+v"(ll));
       load_chunk_px3_nw(smem, wt, 0, krows, a.c_out, co0, wave, nw, ll);
     }
-    float acc[64];
+    if (SPLIT > 1 && dense && s_queued[tile] != 0u) {
+      walk = false;
+      ybase = yrange;
+    }
+    float acc[CW];
 #pragma unroll
-    for (int co = 0; co < 64; ++co) acc[co] = s_seed[co];
-    __builtin_amdgcn_s_waitcnt(0);
+    for (int co = 0; co < CW; ++co) acc[co] = s_seed[CW * part + co];
+    lds_dma_wait();
     __syncthreads();
     for (int c = 0; c < nchunks; ++c) {
       // Chunk c+1 streams into the other buffer; it was last read during
@@ -603,7 +651,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const
         uint32_t nz = 0u;
 #pragma unroll
         for (int tp = 0; tp < 9; ++tp) nz |= (w[tp] != 0u ? 1u : 0u) << tp;
-        const char* chunk = smem + (c & 1) * LY::chunk_bytes;
+        const char* chunk = smem + (c & 1) * LY::chunk_bytes + CW * 4 * part;
         uint32_t m = 0u;
         const char* trows = chunk;
         // Per-lane cursor over (tap, ci): the wavefront loops while any
@@ -627,10 +675,10 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const
             // products wait for the next chunk's rows and words too.
             __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
           }
-          px3_add_row_at<64>(acc, px3_spike_row(trows, bit), 0, xv);
+          px3_add_pieces<CW>(acc, px3_spike_row(trows, bit), xv);
         }
       }
-      __builtin_amdgcn_s_waitcnt(0);
+      lds_dma_wait();
       __syncthreads();
     }
     {
@@ -638,12 +686,12 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const
       // without a pixel start at its end; channels past C_out are skipped.
       int hwo_t = hwo, c_out_t = a.c_out;
       asm volatile("" : "+s"(hwo_t), "+s"(c_out_t));
-      const int nco = min(64, c_out_t - co0);
+      const int nco = min(CW, c_out_t - co0 - CW * part);
       const auto rs = buf_rsrc(y, yrange);
       const uint32_t plane = (uint32_t)hwo_t * B;
       uint32_t off = ybase;
 #pragma unroll
-      for (int co = 0; co < 64; ++co) {
+      for (int co = 0; co < CW; ++co) {
         if (co < nco) BufIO<TOut>::store(from_f32<TOut>(acc[co]), rs, (int)off, 0);
         off += plane;
         asm volatile("" : "+v"(off));
@@ -997,24 +1045,29 @@ int launch_px3_t(const ConvArgs& a, int out_dtype, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 
-template <typename TIn, typename TOut>
-int launch_px3s_to(const ConvArgs& a, hipStream_t stream, DenseQueue** dense) {
+template <typename TIn, typename TOut, int CW>
+int launch_px3s_cw(const ConvArgs& a, int groups, int64_t tiles, int nt, hipStream_t stream, DenseQueue* dq) {
   typedef Px3Layout<64> LY;
-  const int groups = (a.c_out + 63) / 64;
   const int nchunks = (a.c_in + kPx3Ch - 1) / kPx3Ch;
-  const int64_t tiles = (a.n * (int64_t)a.hw_out + 63) / 64;
-  const int nw = even_pass_waves(tiles * groups);
-  const int64_t per_group = (tiles + nw - 1) / nw;
-  const int grid = (int)(groups * per_group);
-  constexpr auto kern = k_conv_px3s<TIn, TOut>;
+  const int grid = (int)(groups * ((tiles + nt - 1) / nt));
+  constexpr auto kern = k_conv_px3s<TIn, TOut, CW>;
   const int e = set_lds_limit_once<kern>(kMaxLdsBytes - 1024);
   if (e != (int)hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kRowsWaves), (size_t)2 * LY::chunk_bytes, stream, a, a.bits, a.flags,
+                     static_cast<const TIn*>(a.x), a.wt, a.bias, static_cast<TOut*>(a.y), groups, nchunks, nt, dq);
+  return (int)hipGetLastError();
+}
+
+template <typename TIn, typename TOut>
+int launch_px3s_to(const ConvArgs& a, hipStream_t stream, DenseQueue** dense) {
+  const int groups = (a.c_out + 63) / 64;
+  const int64_t tiles = (a.n * (int64_t)a.hw_out + 63) / 64;
+  const int nt = even_pass_waves(tiles * groups);
   // (Queue entries hold a run's first pixel of the flattened axis in 31 bits.)
   DenseQueue* dq =
       groups <= kDenseQueueGroups && a.n * (int64_t)a.hw_out < (1ll << 31) ? dense_queue_for(stream) : nullptr;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * nw), (size_t)2 * LY::chunk_bytes, stream, a, a.bits, a.flags,
-                     static_cast<const TIn*>(a.x), a.wt, a.bias, static_cast<TOut*>(a.y), groups, nchunks, dq);
-  const int rc = (int)hipGetLastError();
+  const int rc = nt <= kPx3sSplitTiles ? launch_px3s_cw<TIn, TOut, 16>(a, groups, tiles, nt, stream, dq)
+                                       : launch_px3s_cw<TIn, TOut, 64>(a, groups, tiles, nt, stream, dq);
   if (rc == (int)hipSuccess) *dense = dq;
   return rc;
 }

@@ -35,7 +35,7 @@ __device__ __forceinline__ void load_chunk(char* buf, const float* __restrict__ 
       const int row = c * (32 * 9) + u * 4 + (lane >> 4);
       const int col = co0 + 4 * (lane & 15);
       const float* src = (row < krows && col < c_out) ? wt + (int64_t)row * c_out + col : wt;
-      __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)(buf + u * 1024), 16, 0, 0);
+      lds_dma16(src, buf + u * 1024);
     }
   }
 }
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_rows_kc(ConvArgs a, co
 
   if (resident) {
     for (int c = 0; c < nchunks; ++c) load_chunk(smem + c * kChunkBytes, wt, c, krows, a.c_out, co0, wave, lane);
-    __builtin_amdgcn_s_waitcnt(0);
+    lds_dma_wait();
     __syncthreads();
   }
   // Passes of kRowsWaves tiles.  With more than two chunks every wavefront
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_rows_kc(ConvArgs a, co
     if (!resident) {
       __syncthreads();  // the previous pass is done with both buffers
       load_chunk(smem, wt, 0, krows, a.c_out, co0, wave, lane);
-      __builtin_amdgcn_s_waitcnt(0);
+      lds_dma_wait();
       __syncthreads();
     }
     for (int c = 0; c < nchunks; ++c) {
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_rows_kc(ConvArgs a, co
         kc_rows<TH, W, 0>(acc, k);
       }
       if (!resident) {
-        __builtin_amdgcn_s_waitcnt(0);
+        lds_dma_wait();
         __syncthreads();
       }
     }

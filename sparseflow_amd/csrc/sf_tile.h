@@ -189,6 +189,29 @@ __device__ __forceinline__ int xcd_range_block(int i, int n) {
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __attribute__((address_space(1))) void* gbl_ptr_t;
 
+// 16 (or 4) bytes per lane from src to LDS address dst + 16 (4) * lane, for
+// loads that run beside the walk of another buffer.  In asm: behind the
+// builtin of the same instruction the compiler puts s_waitcnt vmcnt(0) before
+// the next LDS read, whichever buffer it reads, so the loads would be waited
+// for at once.  It does not count these: the caller waits (lds_dma_wait)
+// before the barrier that hands the buffer over.  Its own counted waits only
+// become longer by them.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 in the clobber list
+__device__ __forceinline__ void lds_dma16(const void* src, void* dst) {
+  const uint32_t l = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)dst);
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(l) : "m0", "memory");
+}
+__device__ __forceinline__ void lds_dma4(const void* src, void* dst) {
+  const uint32_t l = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)dst);
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(l) : "m0", "memory");
+}
+#pragma clang diagnostic pop
+__device__ __forceinline__ void lds_dma_wait() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0);  // tells the compiler that its own loads have landed too
+}
+
 // OR of the non-binary chunk flags covering input rows ih_a .. ih_b (clamped
 // to the frame).
 __device__ __forceinline__ bool rows_value_path(const ConvArgs& a, const uint32_t* __restrict__ flags, int64_t frame,

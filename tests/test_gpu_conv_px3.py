@@ -290,3 +290,32 @@ def test_px3_random_shapes(case):
     assert torch.equal(y1, y2)
     ok, err, _ = close(y1, oconv.sparse_conv2d_ref(x, w, b, s, 1), **FP32_TOL)
     assert ok, f"max abs err {err}"
+
+
+# C_in > 128 on the flattened tiles, by the tiles a workgroup gets on 256 CUs:
+# one tile of one lane; one to four (each walked by four wavefronts, 16
+# channels each) and five (one wavefront, 64); channel groups that end inside
+# a wavefront's 16; dense tiles beside walked ones.
+SPLIT_CASES = [(1, 132, 1, 1, 20, 1), (2, 160, 5, 13, 4, 1), (64, 129, 16, 16, 64, 1), (65, 140, 16, 16, 76, 1),
+               (200, 136, 16, 16, 84, 1), (129, 150, 23, 22, 64, 2), (321, 130, 16, 16, 60, 1)]
+
+
+@pytest.mark.parametrize("case", SPLIT_CASES)
+@pytest.mark.parametrize("form", ["sparse", "dense tiles", "values"])
+def test_px3_streamed_tiles_split_over_wavefronts(case, form):
+    N, C, H, W, Co, s = case
+    announce(f"px3 split {case} {form}")
+    g = torch.Generator(device=DEV).manual_seed(N + C)
+    x = (torch.rand(N, C, H, W, generator=g, device=DEV) < 0.01).float()
+    if form == "dense tiles":
+        x[::3] = (torch.rand(x[::3].shape, generator=g, device=DEV) < 0.3).float()
+    elif form == "values":
+        x[0] *= 0.7
+    w, b = _weights(Co, C).to(DEV), torch.linspace(-0.3, 0.3, Co, device=DEV)
+    y, kernels = _run(x, w, b, s)
+    assert "conv_px3" in kernels, kernels
+    ref = torch.nn.functional.conv2d(x.cpu().double(), w.cpu().double(), b.cpu().double(), stride=s, padding=1)
+    # Walked sums round once per spike at 2^-24, dense tiles lose 2^-16 of |W|.
+    bound = 2.0 ** -15 * torch.nn.functional.conv2d(x.cpu().double(), w.cpu().double().abs(), None, s, 1) + 1e-6
+    assert bool(((y.cpu().double() - ref).abs() <= bound).all())
+    assert torch.equal(y, _run(x, w, b, s)[0])
