@@ -44,6 +44,25 @@ namespace {
 constexpr int kPx3Ch = 32;               // input channels per chunk (one bitmap word)
 constexpr int kPx3Rows = kPx3Ch * 9;     // weight rows per chunk
 
+// Up to this many tiles per workgroup, four wavefronts walk a tile, a quarter
+// of its output channels each (the same sums in the same order), in k_conv_px3s
+// and k_conv_px3w; in every one of these kernels wavefronts up to kRowsWaves
+// that have no tile load weights.  A tile's walk and, with few wavefronts, the
+// weight loads are serial chains that nothing else on the CU hides.  us, one
+// loading and walking wavefront per tile -> 16 loading -> four walking:
+//   streamed   74 x 509 x 8 x 7 -> 48 (clustered spikes)  187 -> 69 -> 48
+//              98 x 451 x 19 x 18 -> 40                   157 -> 124 -> 84
+//              101 x 144 x 15 x 15 -> 52                  46.8 -> 31 -> 23
+//              10 x 191 x 8 x 8 -> 60                     70 -> 27 -> 22
+//   resident   12 x 83 x 17 x 16 -> 36                    22.0 -> 13.7 -> 12.4
+//              52 x 21 x 11 x 10 -> 208                   14.6 -> 8.9 -> 8.2
+//   fused LIF  8 x 4 x 34 x 8 x 8 -> 112                  87.8 -> 76.7 -> 39.8
+//              4 x 8 x 128 x 28 x 28 -> 128               55.2 -> 50.3 -> 30.9
+// Five to eight tiles walked by two wavefronts each gain nothing (streamed, 512
+// x 512 x 14 x 14 -> 512 stride 2 152.6 / 152.1, 158 x 319 x 44 x 44 -> 52 120 /
+// 115).
+constexpr int kPx3SplitTiles = 4;
+
 // LDS layout of a chunk for a workgroup slice of CO output channels.
 //  CO = 64: rows of 16 pieces (16 bytes = 4 channels) padded to 17 pieces
 //           (272 bytes), read at immediate offsets.
@@ -139,6 +158,24 @@ __device__ __forceinline__ void px3_add_pieces(float (&acc)[CW], const char* row
       acc[4 * s + 2] = fmaf(xv, v[s].z, acc[4 * s + 2]);
       acc[4 * s + 3] = fmaf(xv, v[s].w, acc[4 * s + 3]);
     }
+  }
+}
+
+// CW channels of row r of the 32-channel layout from piece p0 on, times xv.
+template <int CW>
+__device__ __forceinline__ void px3_add_swizzled(float (&acc)[CW], const char* chunk, int r, int p0, float xv) {
+  typedef Px3Layout<32> L;
+  const char* rowp = chunk + (r * L::stride) * 16;
+  const int key = ((r >> 1) & L::xmask) << 4;
+  float4 v[CW / 4];
+#pragma unroll
+  for (int s = 0; s < CW / 4; ++s) v[s] = *reinterpret_cast<const float4*>(rowp + (((p0 + s) << 4) ^ key));
+#pragma unroll
+  for (int s = 0; s < CW / 4; ++s) {
+    acc[4 * s] = fmaf(xv, v[s].x, acc[4 * s]);
+    acc[4 * s + 1] = fmaf(xv, v[s].y, acc[4 * s + 1]);
+    acc[4 * s + 2] = fmaf(xv, v[s].z, acc[4 * s + 2]);
+    acc[4 * s + 3] = fmaf(xv, v[s].w, acc[4 * s + 3]);
   }
 }
 
@@ -290,7 +327,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3(ConvArgs a, const 
                                                               const float* __restrict__ wt,
                                                               const float* __restrict__ bias_p,
                                                               void* __restrict__ y, int groups, int nchunks,
-                                                              int out_dtype) {
+                                                              int out_dtype, int nt) {
   typedef Px3Layout<CO> LY;
   extern __shared__ __align__(16) char smem[];
   const int lane0 = lane_id();
@@ -334,18 +371,18 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3(ConvArgs a, const 
   uint32_t wn[9];
   if constexpr (!LIF) {
     int ih0, iw0, sample;
-    if (px3_tile(a, (blk / groups) * kRowsWaves + wave, lane0, total, tpf, sample, ih0, iw0))
+    if (wave < nt && px3_tile(a, (blk / groups) * nt + wave, lane0, total, tpf, sample, ih0, iw0))
       px3_load_words(wn, bits + (int64_t)sample * a.hw_in * a.cwp, a, ih0, iw0, 0);
   }
-  // Passes of kRowsWaves tiles.  With streamed chunks every wavefront takes
-  // part in every barrier, including those of a pass past the end.
-  for (int pass = blk / groups; pass * kRowsWaves < total; pass += nblk) {
+  // Passes of nt tiles, a wavefront each.  With streamed chunks every wavefront
+  // takes part in every load and barrier, also one without a tile.
+  for (int pass = blk / groups; pass * nt < total; pass += nblk) {
     // Lane-dependent addresses are recomputed in every pass rather than kept
     // live across the loop (the accumulators need the registers).
     int lane = lane0;
     asm volatile("" : "+v"(lane));
-    const int t = pass * kRowsWaves + wave;
-    const bool valid = t < total;
+    const int t = pass * nt + wave;
+    const bool valid = wave < nt && t < total;
     const int sample = valid ? t / tpf : 0;
     const int p0 = valid ? (t - sample * tpf) * 64 : 0;
     const int npx = min(64, hwo - p0);
@@ -467,7 +504,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3(ConvArgs a, const 
     }
     if constexpr (!LIF) {
       int nih0, niw0, nsample;
-      if (px3_tile(a, (pass + nblk) * kRowsWaves + wave, lane, total, tpf, nsample, nih0, niw0))
+      if (wave < nt && px3_tile(a, (pass + nblk) * nt + wave, lane, total, tpf, nsample, nih0, niw0))
         px3_load_words(wn, bits + (int64_t)nsample * a.hw_in * a.cwp, a, nih0, niw0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -497,18 +534,6 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3(ConvArgs a, const 
 // element (co, oh, ow) = bias[co] + its active taps summed by one lane in
 // (chunk, tap, ci) order, as there.
 // ---------------------------------------------------------------------------
-
-// Up to this many tiles per workgroup, four wavefronts walk a tile, 16 output
-// channels each (the same sums in the same order); wavefronts up to
-// kRowsWaves that have no tile load weights.  A tile's walk and, with few
-// wavefronts, the chunk loads are serial chains that nothing else on the CU
-// hides: 74 x 509 x 8 x 7 -> 48 (clustered spikes, 65 tiles) took 187 us, 141
-// of them loading with one wavefront per CU; loads by 16 wavefronts 69 us,
-// walked by four 48 us.  98 x 451 x 19 x 18 -> 40 157 -> 124 -> 84, 101 x 144 x
-// 15 x 15 -> 52 46.8 -> 31 -> 23, 10 x 191 x 8 x 8 -> 60 70 -> 27 -> 22.  Five to
-// eight tiles walked by two wavefronts each gain nothing (512 x 512 x 14 x 14 ->
-// 512 stride 2 152.6 / 152.1 us, 158 x 319 x 44 x 44 -> 52 120 / 115).
-constexpr int kPx3sSplitTiles = 4;
 
 // Direct-to-LDS loads of chunk c by the nw wavefronts of the workgroup.
 __device__ __forceinline__ void load_chunk_px3_nw(char* buf, const float* __restrict__ wt, int c, int krows,
@@ -731,9 +756,10 @@ constexpr int px3w_bytes() { return CO == 64 ? kPx3wBytes : kPx3w32Bytes; }
 // never used.
 template <int CO>
 __device__ __forceinline__ void load_rows_px3w(char* buf, const float* __restrict__ wt, int krows, int c_out, int co0,
-                                               int wave, int nw, int lane) {
+                                               int wave, int lane) {
   if constexpr (CO == 64) {
-    for (int u = wave; u < kPx3wUnits; u += nw) {
+    const int units = min(kPx3wUnits, (krows * 17 + 63) / 64);  // (rows past krows are not read)
+    for (int u = wave; u < units; u += kRowsWaves) {
       const int pos = u * 64 + lane;
       const int r = pos / 17, q = pos - r * 17;
       const int col = co0 + 4 * q;
@@ -741,7 +767,8 @@ __device__ __forceinline__ void load_rows_px3w(char* buf, const float* __restric
       __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)(buf + u * 1024), 16, 0, 0);
     }
   } else {
-    for (int u = wave; u < kPx3w32Units; u += nw) {
+    const int units = min(kPx3w32Units, (krows * 8 + 63) / 64);
+    for (int u = wave; u < units; u += kRowsWaves) {
       const int pos = u * 64 + lane;
       const int r = pos >> 3, q = pos & 7;
       const int col = co0 + 4 * (q ^ ((r >> 1) & 7));
@@ -790,18 +817,20 @@ __device__ __forceinline__ void px3w_load_words(uint32_t (&lo)[9], uint32_t (&hi
 // membrane stays in acc over the T steps of a tile, each step's spikes are
 // stored as 4-pixel vectors after the next step's first words are
 // requested, and v_T is stored at the end; y is then the spike tensor.
-template <typename TIn, typename TOut, int CO, bool LIF>
+template <typename TIn, typename TOut, int CO, bool LIF, int CW>
 __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3w(ConvArgs a, const uint32_t* __restrict__ bits,
                                                                const uint32_t* __restrict__ flags,
                                                                const TIn* __restrict__ x, const float* __restrict__ wt,
                                                                const float* __restrict__ bias_p, TOut* __restrict__ y,
-                                                               int groups) {
+                                                               int groups, int nt) {
   static_assert(!LIF || CO == 32, "the fused LIF form keeps one spike word per lane");
   extern __shared__ __align__(16) char smem[];
   __shared__ float s_seed[CO];
   const int lane0 = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int nw = __builtin_amdgcn_readfirstlane((int)(blockDim.x >> 6));  // tiles per pass
+  constexpr int SPLIT = CO / CW;
+  const int tile = SPLIT == 1 ? wave : wave / SPLIT;  // of the nt tiles of a pass; past them: a wavefront that only loads
+  const int cw0 = SPLIT == 1 ? 0 : CW * (wave % SPLIT);  // its first channel
   const int blk = groups >= 8 ? xcd_local_block((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
   const int grp = blk % groups;
   const int co0 = grp * CO;
@@ -817,15 +846,15 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3w(ConvArgs a, const
     const float b = (bias_p != nullptr && co < a.c_out) ? bias_p[co] : 0.f;
     s_seed[threadIdx.x] = LIF ? L.vr_term + b : b;
   }
-  load_rows_px3w<CO>(smem, wt, a.c_in * 9, a.c_out, co0, wave, nw, lane0);
+  load_rows_px3w<CO>(smem, wt, a.c_in * 9, a.c_out, co0, wave, lane0);
   // The first tile's words; later tiles' are requested before the previous
   // tile's stores (the vector memory counter retires in issue order).  The
   // fused LIF form requests a tile's first words at the tile and prefetches
   // per step (the T steps of a tile are its long stretch of work).
   uint32_t nlo[9], nhi[9];
   if constexpr (!LIF) {
-    const int t = (blk / groups) * nw + wave;
-    if (t < total) {
+    const int t = (blk / groups) * nt + tile;
+    if (tile < nt && t < total) {
       const int sample = t / tpf, p0 = (t - sample * tpf) * 64;
       const int q = p0 + min(lane0, hwo - p0 - 1);
       const int oh = q / a.w_out, ow = q - oh * a.w_out;
@@ -834,10 +863,11 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3w(ConvArgs a, const
   }
   __builtin_amdgcn_s_waitcnt(0);  // this wavefront's direct weight loads have landed
   __syncthreads();
-  for (int pass = blk / groups; pass * nw < total; pass += nblk) {
+  if (tile >= nt) return;
+  for (int pass = blk / groups; pass * nt < total; pass += nblk) {
     int lane = lane0;
     asm volatile("" : "+v"(lane));
-    const int t = pass * nw + wave;
+    const int t = pass * nt + tile;
     const bool valid = t < total;
     const int sample = valid ? t / tpf : 0;
     const int p0 = valid ? (t - sample * tpf) * 64 : 0;
@@ -848,27 +878,27 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3w(ConvArgs a, const
     const int ih0 = oh * a.s - 1, iw0 = ow * a.s - 1;
     int hwo_t = hwo, c_out_t = a.c_out;
     asm volatile("" : "+s"(hwo_t), "+s"(c_out_t));
-    float acc[CO];
+    float acc[CW];
     if constexpr (LIF) {
       // Membrane before step 0: v_init or 0.
-      const int nco = min(CO, c_out_t - co0);
+      const int nco = min(CW, c_out_t - co0 - cw0);
       const float* vi = a.v_init;
 #pragma unroll
-      for (int co = 0; co < CO; ++co) acc[co] = 0.f;
+      for (int co = 0; co < CW; ++co) acc[co] = 0.f;
       if (vi != nullptr && mine) {
-        const float* vp = vi + ((int64_t)sample * c_out_t + co0) * hwo_t + p0 + lane;
+        const float* vp = vi + ((int64_t)sample * c_out_t + co0 + cw0) * hwo_t + p0 + lane;
 #pragma unroll
-        for (int co = 0; co < CO; ++co)
+        for (int co = 0; co < CW; ++co)
           if (co < nco) acc[co] = vp[(int64_t)co * hwo_t];
       }
       px3w_load_words(nlo, nhi, bits + (int64_t)sample * a.hw_in * a.cwp, a, ih0, iw0, 0);
     } else {
 #pragma unroll
-      for (int co = 0; co < CO; ++co) acc[co] = s_seed[co];
+      for (int co = 0; co < CW; ++co) acc[co] = s_seed[cw0 + co];
     }
     for (int st = 0; st < steps; ++st) {
       const int64_t frame = LIF ? (int64_t)st * a.n + sample : sample;
-      if constexpr (LIF) lif_seed_lds<CO>(acc, L, s_seed);
+      if constexpr (LIF) lif_seed_lds<CW>(acc, L, s_seed + cw0);
       bool value = false;
       if (valid) {
         const int oh_a = p0 / a.w_out, oh_b = (p0 + npx - 1) / a.w_out;
@@ -900,13 +930,13 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3w(ConvArgs a, const
           // lane has spikes left.
           uint64_t m = 0ull;
           int tap = 0;               // CO = 32
-          const char* trows = smem;  // CO = 64: the tap's rows (row0 = 0)
+          const char* trows = smem + 4 * cw0;  // CO = 64: the tap's rows (row0 = 0)
           while ((m != 0ull) || (nz != 0u)) {
             if (m == 0ull) {
               const int t = __builtin_ctz(nz);
               nz &= nz - 1u;
               m = ((uint64_t)px3_select(wh, t) << 32) | px3_select(wl, t);
-              if constexpr (CO == 64) trows = px3_tap_rows(smem, t);
+              if constexpr (CO == 64) trows = px3_tap_rows(smem + 4 * cw0, t);
               else tap = t;
             }
             const int bit = __builtin_ctzll(m);
@@ -918,7 +948,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3w(ConvArgs a, const
                 // The tap and the lane's window origin formed here (the
                 // lane index anew, in asm): kept live across the walk they
                 // take registers the walk needs.
-                tap = px3_rows_tap(smem, trows);
+                tap = px3_rows_tap(smem + 4 * cw0, trows);
                 int ln;
                 asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
                 const int qv = p0 + min(ln, npx - 1);
@@ -935,31 +965,32 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3w(ConvArgs a, const
               // bitmap path too.
               __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
             }
-            if constexpr (CO == 64) px3_add_row_at<64>(acc, px3_spike_row(trows, bit), 0, xv);
-            else px3_add_row<CO, !LIF>(acc, smem, row0 + bit * 9 + tap, xv);
+            if constexpr (CO == 64) px3_add_pieces<CW>(acc, px3_spike_row(trows, bit), xv);
+            else if constexpr (SPLIT == 1) px3_add_row<CO, !LIF>(acc, smem, row0 + bit * 9 + tap, xv);
+            else px3_add_swizzled<CW>(acc, smem, row0 + bit * 9 + tap, cw0 / 4, xv);
           }
         }
       }
       if constexpr (LIF) {
         // Spikes and reset; the next step's first words are requested
         // before the spike stores.
-        const int nco = min(CO, c_out_t - co0);
-        const uint32_t sw = lif_fire<CO>(acc, L);
+        const int nco = min(CW, c_out_t - co0 - cw0);
+        const uint32_t sw = lif_fire<CW>(acc, L);
         if (st + 1 < steps)
           px3w_load_words(nlo, nhi, bits + (frame + a.n) * a.hw_in * a.cwp, a, ih0, iw0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        TOut* __restrict__ spk = y + (frame * c_out_t + co0) * hwo_t;
-        px3_store_spikes<TOut, CO>(sw, spk, lane, p0, npx, valid, mine, nco, hwo_t, c_out_t);
+        TOut* __restrict__ spk = y + (frame * c_out_t + co0 + cw0) * hwo_t;
+        px3_store_spikes<TOut, CW>(sw, spk, lane, p0, npx, valid, mine, nco, hwo_t, c_out_t);
       }
     }
     if constexpr (LIF) {
       if (mine) {
-        const int64_t vb = ((int64_t)sample * c_out_t + co0) * hwo_t + p0 + lane;
-        px3_store<CO>(acc, a.v_out + vb, hwo_t, min(CO, c_out_t - co0));
+        const int64_t vb = ((int64_t)sample * c_out_t + co0 + cw0) * hwo_t + p0 + lane;
+        px3_store<CW>(acc, a.v_out + vb, hwo_t, min(CW, c_out_t - co0 - cw0));
       }
     } else {
       {
-        const int tn = (pass + nblk) * nw + wave;
+        const int tn = (pass + nblk) * nt + tile;
         if (tn < total) {
           const int ns = tn / tpf, np0 = (tn - ns * tpf) * 64;
           const int nq = np0 + min(lane, hwo - np0 - 1);
@@ -974,7 +1005,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3w(ConvArgs a, const
       constexpr uint32_t B = (uint32_t)sizeof(TOut);
       const uint32_t range = (uint32_t)c_out_t * (uint32_t)hwo_t * B;
       const auto rs = buf_rsrc(y + (int64_t)sample * c_out_t * hwo_t, range);
-      const uint32_t base = mine ? ((uint32_t)co0 * (uint32_t)hwo_t + (uint32_t)(p0 + lane)) * B : range;
+      const uint32_t base = mine ? ((uint32_t)(co0 + cw0) * (uint32_t)hwo_t + (uint32_t)(p0 + lane)) * B : range;
       const uint32_t plane = (uint32_t)hwo_t * B;
       // One offset register stepped by a plane per store (opaque, so the
       // offsets are not precomputed into registers); soffset stays 0.
@@ -983,14 +1014,14 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3w(ConvArgs a, const
       uint32_t off = base;
       if ((plane & 127u) == 0u) {
 #pragma unroll
-        for (int co = 0; co < CO; ++co) {
+        for (int co = 0; co < CW; ++co) {
           BufIO<TOut>::template store<kStoreStream>(from_f32<TOut>(acc[co]), rs, (int)off, 0);
           off += plane;
           asm volatile("" : "+v"(off));
         }
       } else {
 #pragma unroll
-        for (int co = 0; co < CO; ++co) {
+        for (int co = 0; co < CW; ++co) {
           BufIO<TOut>::store(from_f32<TOut>(acc[co]), rs, (int)off, 0);
           off += plane;
           asm volatile("" : "+v"(off));
@@ -1000,6 +1031,16 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3w(ConvArgs a, const
   }
 }
 
+template <typename TIn, typename TOut, int CO, bool LIF, int CW>
+int launch_px3w_cw(const ConvArgs& a, int grid, int groups, int nt, hipStream_t stream) {
+  constexpr auto kern = k_conv_px3w<TIn, TOut, CO, LIF, CW>;
+  const int e = set_lds_limit_once<kern>(kMaxLdsBytes - 1024);
+  if (e != (int)hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kRowsWaves), (size_t)px3w_bytes<CO>(), stream, a, a.bits, a.flags,
+                     static_cast<const TIn*>(a.x), a.wt, a.bias, static_cast<TOut*>(a.y), groups, nt);
+  return (int)hipGetLastError();
+}
+
 template <typename TIn, typename TOut, int CO, bool LIF = false>
 int launch_px3w_to(const ConvArgs& a, hipStream_t stream) {
   const int groups = (a.c_out + CO - 1) / CO;
@@ -1007,16 +1048,12 @@ int launch_px3w_to(const ConvArgs& a, hipStream_t stream) {
   // One workgroup per CU (the weights fill the LDS) making the same number
   // of passes: as many as 16-wave workgroups would need, with the wave-tiles
   // spread evenly over them (no CU idles through another's last pass).
-  const int nw = even_pass_waves(tiles * groups);
-  const int64_t passes = (tiles * groups + (int64_t)num_cus() * nw - 1) / ((int64_t)num_cus() * nw);
-  const int64_t per_group = (tiles + (int64_t)nw * passes - 1) / ((int64_t)nw * passes);
+  const int nt = even_pass_waves(tiles * groups);
+  const int64_t passes = (tiles * groups + (int64_t)num_cus() * nt - 1) / ((int64_t)num_cus() * nt);
+  const int64_t per_group = (tiles + (int64_t)nt * passes - 1) / ((int64_t)nt * passes);
   const int grid = (int)(groups * (per_group > 0 ? per_group : 1));
-  constexpr auto kern = k_conv_px3w<TIn, TOut, CO, LIF>;
-  const int e = set_lds_limit_once<kern>(kMaxLdsBytes - 1024);
-  if (e != (int)hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * nw), (size_t)px3w_bytes<CO>(), stream, a, a.bits, a.flags,
-                     static_cast<const TIn*>(a.x), a.wt, a.bias, static_cast<TOut*>(a.y), groups);
-  return (int)hipGetLastError();
+  return nt <= kPx3SplitTiles ? launch_px3w_cw<TIn, TOut, CO, LIF, CO / 4>(a, grid, groups, nt, stream)
+                              : launch_px3w_cw<TIn, TOut, CO, LIF, CO>(a, grid, groups, nt, stream);
 }
 
 template <typename TIn, int CO>
@@ -1034,14 +1071,18 @@ int launch_px3_t(const ConvArgs& a, int out_dtype, hipStream_t stream) {
   const int held = nchunks <= LY::resident_chunks ? nchunks : 2;
   const size_t lds = (size_t)held * LY::chunk_bytes;
   const int64_t tiles = a.n * (int64_t)((a.hw_out + 63) / 64);
-  const int64_t need = (tiles + kRowsWaves - 1) / kRowsWaves;
-  const int per_group = (int)(need < num_cus() ? need : num_cus());
-  const int grid = groups * (per_group > 0 ? per_group : 1);
+  // The tiles spread over the CUs as in launch_px3w_to: full workgroups of 16
+  // left most of them idle (fused LIF, 4 x 8 x 200 x 14 x 14 -> 200: 173 -> 117
+  // us).
+  const int nt = even_pass_waves(tiles * groups);
+  const int64_t passes = (tiles * groups + (int64_t)num_cus() * nt - 1) / ((int64_t)num_cus() * nt);
+  const int64_t per_group = (tiles + (int64_t)nt * passes - 1) / ((int64_t)nt * passes);
+  const int grid = (int)(groups * (per_group > 0 ? per_group : 1));
   constexpr auto kern = k_conv_px3<TIn, TOut, CO, LIF>;
   const int e = set_lds_limit_once<kern>(kMaxLdsBytes - 1024);
   if (e != (int)hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kRowsWaves), lds, stream, a, a.bits, a.flags,
-                     static_cast<const TIn*>(a.x), a.wt, a.bias, a.y, groups, nchunks, out_dtype);
+                     static_cast<const TIn*>(a.x), a.wt, a.bias, a.y, groups, nchunks, out_dtype, nt);
   return (int)hipGetLastError();
 }
 
@@ -1066,7 +1107,7 @@ int launch_px3s_to(const ConvArgs& a, hipStream_t stream, DenseQueue** dense) {
   // (Queue entries hold a run's first pixel of the flattened axis in 31 bits.)
   DenseQueue* dq =
       groups <= kDenseQueueGroups && a.n * (int64_t)a.hw_out < (1ll << 31) ? dense_queue_for(stream) : nullptr;
-  const int rc = nt <= kPx3sSplitTiles ? launch_px3s_cw<TIn, TOut, 16>(a, groups, tiles, nt, stream, dq)
+  const int rc = nt <= kPx3SplitTiles ? launch_px3s_cw<TIn, TOut, 16>(a, groups, tiles, nt, stream, dq)
                                        : launch_px3s_cw<TIn, TOut, 64>(a, groups, tiles, nt, stream, dq);
   if (rc == (int)hipSuccess) *dense = dq;
   return rc;

@@ -292,17 +292,19 @@ def test_px3_random_shapes(case):
     assert ok, f"max abs err {err}"
 
 
-# C_in > 128 on the flattened tiles, by the tiles a workgroup gets on 256 CUs:
-# one tile of one lane; one to four (each walked by four wavefronts, 16
-# channels each) and five (one wavefront, 64); channel groups that end inside
-# a wavefront's 16; dense tiles beside walked ones.
+# The tiles a workgroup gets on 256 CUs: one tile of one lane; one to four (each
+# walked by four wavefronts, a quarter of the channels each) and five and more
+# (one wavefront); channel groups that end inside a wavefront's quarter; dense
+# tiles beside walked ones.  C_in > 128 (streamed), up to 128 and up to 64.
 SPLIT_CASES = [(1, 132, 1, 1, 20, 1), (2, 160, 5, 13, 4, 1), (64, 129, 16, 16, 64, 1), (65, 140, 16, 16, 76, 1),
-               (200, 136, 16, 16, 84, 1), (129, 150, 23, 22, 64, 2), (321, 130, 16, 16, 60, 1)]
+               (200, 136, 16, 16, 84, 1), (129, 150, 23, 22, 64, 2), (321, 130, 16, 16, 60, 1),
+               (1, 100, 1, 1, 20, 1), (2, 128, 5, 13, 36, 1), (64, 65, 16, 16, 64, 1), (200, 100, 15, 14, 76, 2),
+               (1, 20, 1, 1, 4, 1), (2, 40, 5, 13, 20, 1), (65, 64, 16, 16, 76, 1), (321, 33, 16, 16, 60, 1)]
 
 
 @pytest.mark.parametrize("case", SPLIT_CASES)
 @pytest.mark.parametrize("form", ["sparse", "dense tiles", "values"])
-def test_px3_streamed_tiles_split_over_wavefronts(case, form):
+def test_px3_tiles_split_over_wavefronts(case, form):
     N, C, H, W, Co, s = case
     announce(f"px3 split {case} {form}")
     g = torch.Generator(device=DEV).manual_seed(N + C)

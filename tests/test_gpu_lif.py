@@ -241,3 +241,22 @@ def test_fused_lif_pixel_kernel_random_shapes(case):
         x.to(DEV), w.to(DEV), b.to(DEV), tau=2.0, v_threshold=1.0, v_reset=v_reset, decay_input=decay_input))
     assert "conv_lif_px3" in kernels, kernels
     _check(spk, v, x, w, b, 3, 2.0, 1.0, v_reset, decay_input)
+
+
+# Tiles per workgroup as the pixel kernel spreads them over 256 CUs: one to
+# four (four wavefronts per tile where the weights stay resident, C_in <= 128)
+# and more; channel slices that end inside a wavefront's eight.
+SPREAD_CASES = [(3, 1, 20, 3, 5, 4), (2, 2, 128, 9, 13, 36), (2, 96, 64, 16, 16, 44), (2, 190, 33, 16, 14, 64),
+                (2, 2, 132, 9, 13, 36), (2, 96, 150, 16, 16, 44)]
+
+
+@pytest.mark.parametrize("case", SPREAD_CASES)
+def test_fused_lif_tiles_spread_over_cus(case):
+    T, N, C, H, W, Co = case
+    announce(f"lif spread {case}")
+    x = spikes((T, N, C, H, W), 0.05, seed=N + C)
+    w = torch.randn(Co, C, 3, 3, generator=torch.Generator().manual_seed(C)) * (4.0 / (C * 9)) ** 0.5 * 2.0
+    b = torch.linspace(-0.2, 0.4, Co)
+    spk, v, _ = sparse_fused_conv_lif_multistep(x.to(DEV), w.to(DEV), b.to(DEV), kernel_size=3)
+    torch.cuda.synchronize()
+    _check(spk, v, x, w, b, 3, 2.0, 1.0, 0.0, True)
