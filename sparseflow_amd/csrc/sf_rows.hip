@@ -174,7 +174,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_rows_kc(ConvArgs a, co
                                                                   const float* __restrict__ wt,
                                                                   const float* __restrict__ bias_p,
                                                                   void* __restrict__ y, int groups, int nchunks,
-                                                                  int in_dtype, int out_dtype,
+                                                                  int in_dtype, int out_dtype, int nt,
                                                                   DenseQueue* __restrict__ dq) {
   // Launched only for planes with h*w % 4 == 0, so every tile's run (TH*W, or
   // an even number of 14-wide rows for the last tile) is whole quads.
@@ -199,11 +199,11 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_rows_kc(ConvArgs a, co
     lds_dma_wait();
     __syncthreads();
   }
-  // Passes of kRowsWaves tiles.  With more than two chunks every wavefront
-  // takes part in every barrier, including those of a pass past the end.
-  for (int pass = (blk / groups); pass * kRowsWaves < total; pass += nblk) {
-    const int t = pass * kRowsWaves + wave;
-    const bool valid = t < total;
+  // Passes of nt tiles, a wavefront each.  With more than two chunks every
+  // wavefront takes part in every load and barrier, also one without a tile.
+  for (int pass = (blk / groups); pass * nt < total; pass += nblk) {
+    const int t = pass * nt + wave;
+    const bool valid = wave < nt && t < total;
     const int frame = valid ? t / tpf : 0;
     const int oh0 = valid ? (t - frame * tpf) * TH : 0;
     float acc[64];
@@ -288,9 +288,14 @@ int launch_kc_t(const ConvArgs& a, int in_dtype, int out_dtype, hipStream_t stre
   const int nchunks = (a.c_in + 31) / 32;
   const size_t lds = (size_t)2 * kChunkBytes;
   const int64_t tiles = a.n * (int64_t)((a.h_out + TH - 1) / TH);
-  const int64_t need = (tiles + kRowsWaves - 1) / kRowsWaves;
-  const int per_group = (int)(need < num_cus() ? need : num_cus());
-  const int grid = groups * (per_group > 0 ? per_group : 1);
+  // As many tiles per workgroup as spread them evenly over the CUs: full
+  // workgroups of 16 leave most CUs idle at small batches (us, 4 / 16 / 64 x 256
+  // x 14 x 14 -> 256: 49.7 -> 37.7, 51.2 -> 39.3, 53.1 -> 43.8; 16 x 256 x 28 x 28 ->
+  // 256 60.2 -> 50.4; 512 x 256 x 14 x 14 -> 256, full either way, 106.6 / 104.5).
+  const int nt = even_pass_waves(tiles * groups);
+  const int64_t passes = (tiles * groups + (int64_t)num_cus() * nt - 1) / ((int64_t)num_cus() * nt);
+  const int64_t per_group = (tiles + (int64_t)nt * passes - 1) / ((int64_t)nt * passes);
+  const int grid = (int)(groups * (per_group > 0 ? per_group : 1));
   constexpr auto kern = k_conv_rows_kc<TH, W>;
   const int e = set_lds_limit_once<kern>(kMaxLdsBytes);
   if (e != (int)hipSuccess) return e;
@@ -298,7 +303,7 @@ int launch_kc_t(const ConvArgs& a, int in_dtype, int out_dtype, hipStream_t stre
   DenseQueue* dq =
       groups <= kDenseQueueGroups && a.n * (int64_t)a.hw_out < (1ll << 31) ? dense_queue_for(stream) : nullptr;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kRowsWaves), lds, stream, a, a.bits, a.flags, a.x, a.wt, a.bias,
-                     a.y, groups, nchunks, in_dtype, out_dtype, dq);
+                     a.y, groups, nchunks, in_dtype, out_dtype, nt, dq);
   const int rc = (int)hipGetLastError();
   if (rc == (int)hipSuccess) *dense = dq;
   return rc;

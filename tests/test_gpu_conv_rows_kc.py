@@ -123,3 +123,21 @@ def test_rows_kc_deterministic_bitwise():
     y1, _ = _run(x, w, None)
     y2, _ = _run(x, w, None)
     assert torch.equal(y1, y2)
+
+
+# Tiles per workgroup as they spread over 256 CUs: 1 (a frame alone), 1, 4, 7
+# and 16, with the last workgroup's short.
+SPREAD_CASES = [(1, 130, 2, 28, 4), (3, 150, 14, 14, 64), (100, 130, 14, 14, 132), (64, 140, 28, 28, 68),
+                (290, 129, 28, 28, 60)]
+
+
+@pytest.mark.parametrize("case", SPREAD_CASES)
+def test_rows_kc_tiles_spread_over_cus(case):
+    N, C, H, W, Co = case
+    announce(f"rows_kc spread {case}")
+    x = spikes((N, C, H, W), 0.01, seed=N + C)
+    w, b = _weights(Co, C), torch.linspace(-0.3, 0.3, Co)
+    y, kernels = _run(x.to(DEV), w.to(DEV), b.to(DEV))
+    assert "conv_rows_kc" in kernels, kernels
+    ok, err, _ = close(y, oconv.sparse_conv2d_ref(x, w, b, 1, 1), **FP32_TOL)
+    assert ok, f"max abs err {err}"
