@@ -59,7 +59,7 @@ __device__ __forceinline__ void load_chunk_px(char* buf, const float* __restrict
       const int row = c * kPxChunkCh + r;
       const int col = co0 + 4 * piece;
       const float* src = (row < c_in && col < c_out) ? wt + (int64_t)row * c_out + col : wt;
-      lds_dma16(src, buf + u * 1024);
+      __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)(buf + u * 1024), 16, 0, 0);
     }
   }
 }
@@ -75,7 +75,7 @@ __device__ __forceinline__ void load_chunk_px_nw(char* buf, const float* __restr
     const int row = c * kPxChunkCh + r;
     const int col = co0 + 4 * piece;
     const float* src = (row < c_in && col < c_out) ? wt + (int64_t)row * c_out + col : wt;
-    lds_dma16(src, buf + u * 1024);
+    __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)(buf + u * 1024), 16, 0, 0);
   }
 }
 
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_flat(ConvArgs a, const
   if (resident) {
     for (int c = 0; c < nchunks; ++c)
       load_chunk_px_nw(smem + c * kPxChunkBytes, wt, c, a.c_in, a.c_out, co0, wave, nw, lane);
-    lds_dma_wait();
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
   }
   // Passes of nw tiles.  With more than two chunks every wavefront takes
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_flat(ConvArgs a, const
     if (!resident) {
       __syncthreads();  // the previous pass is done with both buffers
       load_chunk_px_nw(smem, wt, 0, a.c_in, a.c_out, co0, wave, nw, lane);
-      lds_dma_wait();
+      __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
     }
     for (int c = 0; c < nchunks; ++c) {
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_flat(ConvArgs a, const
         }
       }
       if (!resident) {
-        lds_dma_wait();
+        __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
       }
     }
@@ -359,7 +359,7 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(XV ? 2
   if (resident) {
     for (int c = 0; c < nchunks; ++c)
       load_chunk_px<NWV>(smem + c * kPxChunkBytes, wt, c, a.c_in, a.c_out, co0, wave, lane0);
-    lds_dma_wait();
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
   }
   for (int pass = (blk / groups); pass * NWV < total; pass += nblk) {
@@ -439,7 +439,7 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(XV ? 2
         int ll = lane;
         asm volatile("" : "+v"(ll));
         load_chunk_px<NWV>(smem, wt, 0, a.c_in, a.c_out, co0, wave, ll);
-        lds_dma_wait();
+        __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
       }
       for (int c = 0; c < nchunks; ++c) {
@@ -477,7 +477,7 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(XV ? 2
           }
         }
         if (!resident) {
-          lds_dma_wait();
+          __builtin_amdgcn_s_waitcnt(0);
           __syncthreads();
         }
       }
