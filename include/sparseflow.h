@@ -422,6 +422,17 @@ int sf_spike_attention(const void* q, const void* k, const void* v,
                        float threshold, void* y, const int64_t* y_strides,
                        int32_t out_dtype, void* stream);
 
+/* ---- launch plans (host only) --------------------------------------------- */
+
+/* How sf_conv2d_sparse (fused_lif = 0) or sf_conv_lif_forward (1) launches the
+ * 3x3 kernels that deal wave-sized output tiles out over workgroups (the
+ * pixel-tile and row-tile kernels): the workgroups, the tiles a workgroup takes
+ * in a pass, and the wavefronts that walk a tile.  One of these workgroups
+ * fills a CU.  SF_ERR_UNSUPPORTED where another kernel runs. */
+int sf_conv2d_launch_plan(const sf_conv_desc* desc, int32_t fused_lif,
+                          int32_t* workgroups, int32_t* tiles,
+                          int32_t* waves_per_tile);
+
 /* ---- per-kernel timing (bench instrumentation) --------------------------- */
 
 /* When enabled, every kernel launched by the library is bracketed by a

@@ -50,6 +50,7 @@ EXPORTS = {
     ),
     "sf_conv2d_sparse": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P]),
     "sf_conv2d_bitmap_layout": (c_int, [_P]),
+    "sf_conv2d_launch_plan": (c_int, [_P, c_int32, _P, _P, _P]),
     "sf_conv2d_sparse_layout": (c_int, [_P, _P, c_int32, _P, _P, _P, _P, _P, _P]),
     "sf_conv2d_forward": (c_int, [_P, _P, _P, _P, c_float, _P, c_size_t, _P, _P]),
     "sf_conv2d_forward_noalloc": (c_int, [_P, _P, _P, _P, c_float, _P, _P]),
@@ -303,6 +304,15 @@ def conv2d_bitmap_layout(desc: ConvDesc) -> int:
     if rc < 0:
         _check(-rc, "sf_conv2d_bitmap_layout")
     return rc
+
+
+def conv2d_launch_plan(desc: ConvDesc, fused_lif: bool = False) -> Tuple[int, int, int]:
+    """(workgroups, tiles of a pass, wavefronts per tile) of the 3x3
+    pixel-tile and row-tile kernels (sf_conv2d_launch_plan)."""
+    out = (c_int32 * 3)()
+    p = [ctypes.byref(out, 4 * i) for i in range(3)]
+    _check(int(lib().sf_conv2d_launch_plan(ctypes.byref(desc), 1 if fused_lif else 0, *p)), "sf_conv2d_launch_plan")
+    return out[0], out[1], out[2]
 
 
 def conv2d_forward(desc: ConvDesc, x: torch.Tensor, wt: torch.Tensor, bias: Optional[torch.Tensor],

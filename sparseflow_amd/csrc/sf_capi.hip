@@ -422,6 +422,25 @@ int sf_conv2d_bitmap_layout(const sf_conv_desc* d) {
   return reads_planes(pick_stage2(d, a)) ? SF_BITMAP_PLANES : SF_BITMAP_PIXEL_MAJOR;
 }
 
+int sf_conv2d_launch_plan(const sf_conv_desc* d, int32_t fused_lif, int32_t* workgroups, int32_t* tiles,
+                          int32_t* waves_per_tile) {
+  const int rc = check_desc(d, fused_lif == 0);
+  if (rc != SF_OK) return rc;
+  if (workgroups == nullptr || tiles == nullptr || waves_per_tile == nullptr) return fail(SF_ERR_INVALID, "NULL pointer");
+  if (d->n == 0) return fail(SF_ERR_UNSUPPORTED, "no frames: nothing is launched");
+  const sf::ConvArgs a = conv_args(d, d->n, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, fused_lif != 0);
+  sf::LaunchPlan p{};
+  const Stage2 k = fused_lif != 0 ? (d->stride == 1 && sf::px3_applicable(a) ? Stage2::kPx3 : Stage2::kGather)
+                                  : pick_stage2(d, a);
+  if (k == Stage2::kPx3) p = sf::px3_plan(a, d->out_dtype, fused_lif != 0);
+  else if (k == Stage2::kRowsKc) p = sf::rows_kc_plan(a);
+  else return fail(SF_ERR_UNSUPPORTED, "this shape's kernel does not spread wave-tiles over channel groups");
+  *workgroups = p.workgroups;
+  *tiles = p.tiles;
+  *waves_per_tile = p.waves_per_tile;
+  return SF_OK;
+}
+
 int sf_conv2d_sparse_layout(const sf_conv_desc* d, const uint32_t* bits, int32_t layout, const uint32_t* flags,
                             const void* x, const float* wt, const float* bias, void* y, void* stream) {
   if (layout != SF_BITMAP_PIXEL_MAJOR && layout != SF_BITMAP_PLANES) return fail(SF_ERR_INVALID, "unknown bitmap layout");

@@ -105,8 +105,15 @@ int launch_conv_band(const ConvArgs& a, int in_dtype, int out_dtype, hipStream_t
 bool rows_fused_applicable(const ConvArgs& a);
 int launch_conv_rows_fused(const ConvArgs& a, int in_dtype, int out_dtype, float cutoff, hipStream_t stream);
 
+// What a launch over wave-tiles looks like: its workgroups, the tiles one of
+// them takes in a pass and the wavefronts that walk a tile.
+struct LaunchPlan {
+  int workgroups, tiles, waves_per_tile;
+};
+
 // K-chunked row-tile Stage 2 (3x3 s1, any C_in, frame width 28 or 14).
 bool rows_kc_applicable(const ConvArgs& a);
+LaunchPlan rows_kc_plan(const ConvArgs& a);
 int launch_conv_rows_kc(const ConvArgs& a, int in_dtype, int out_dtype, hipStream_t stream);
 
 // Flat-tile Stage 2 for 1x1 stride-1 convolutions (any C_in, C_out % 4 == 0).
@@ -118,6 +125,8 @@ bool px3_applicable(const ConvArgs& a);
 // The weights stay resident in LDS for the whole launch (C_in <= 128).
 bool px3_resident(const ConvArgs& a);
 int launch_conv_px3(const ConvArgs& a, int in_dtype, int out_dtype, hipStream_t stream);
+// Its launch (lif: launch_conv_lif_px3's).
+LaunchPlan px3_plan(const ConvArgs& a, int out_dtype, bool lif);
 // Matrix-core Stage 2 for 3x3 layers with a reduction of at most 32
 // (C_in * 9 <= 32, f32 input): the whole K is one dense tile.
 bool mfma_conv_applicable(const ConvArgs& a);

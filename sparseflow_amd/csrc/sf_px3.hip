@@ -1031,6 +1031,17 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3w(ConvArgs a, const
   }
 }
 
+// Frame by frame in 64-pixel tiles (px3, px3w), CO channels to a group.
+template <int CO>
+GroupSpread px3_spread(const ConvArgs& a) {
+  return spread_passes(a.n * (int64_t)((a.hw_out + 63) / 64), (a.c_out + CO - 1) / CO);
+}
+
+// Over the flattened (frame, pixel) axis (px3s).
+GroupSpread px3s_spread(const ConvArgs& a) {
+  return spread_rounds((a.n * (int64_t)a.hw_out + 63) / 64, (a.c_out + 63) / 64);
+}
+
 template <typename TIn, typename TOut, int CO, bool LIF, int CW>
 int launch_px3w_cw(const ConvArgs& a, int grid, int groups, int nt, hipStream_t stream) {
   constexpr auto kern = k_conv_px3w<TIn, TOut, CO, LIF, CW>;
@@ -1044,14 +1055,10 @@ int launch_px3w_cw(const ConvArgs& a, int grid, int groups, int nt, hipStream_t 
 template <typename TIn, typename TOut, int CO, bool LIF = false>
 int launch_px3w_to(const ConvArgs& a, hipStream_t stream) {
   const int groups = (a.c_out + CO - 1) / CO;
-  const int64_t tiles = a.n * (int64_t)((a.hw_out + 63) / 64);
   // One workgroup per CU (the weights fill the LDS) making the same number
-  // of passes: as many as 16-wave workgroups would need, with the wave-tiles
-  // spread evenly over them (no CU idles through another's last pass).
-  const int nt = even_pass_waves(tiles * groups);
-  const int64_t passes = (tiles * groups + (int64_t)num_cus() * nt - 1) / ((int64_t)num_cus() * nt);
-  const int64_t per_group = (tiles + (int64_t)nt * passes - 1) / ((int64_t)nt * passes);
-  const int grid = (int)(groups * (per_group > 0 ? per_group : 1));
+  // of passes: no CU idles through another's last pass.
+  const GroupSpread sp = px3_spread<CO>(a);
+  const int grid = groups * sp.per_group, nt = sp.waves;
   return nt <= kPx3SplitTiles ? launch_px3w_cw<TIn, TOut, CO, LIF, CO / 4>(a, grid, groups, nt, stream)
                               : launch_px3w_cw<TIn, TOut, CO, LIF, CO>(a, grid, groups, nt, stream);
 }
@@ -1070,14 +1077,11 @@ int launch_px3_t(const ConvArgs& a, int out_dtype, hipStream_t stream) {
   const int nchunks = (a.c_in + kPx3Ch - 1) / kPx3Ch;
   const int held = nchunks <= LY::resident_chunks ? nchunks : 2;
   const size_t lds = (size_t)held * LY::chunk_bytes;
-  const int64_t tiles = a.n * (int64_t)((a.hw_out + 63) / 64);
   // The tiles spread over the CUs as in launch_px3w_to: full workgroups of 16
   // left most of them idle (fused LIF, 4 x 8 x 200 x 14 x 14 -> 200: 173 -> 117
   // us).
-  const int nt = even_pass_waves(tiles * groups);
-  const int64_t passes = (tiles * groups + (int64_t)num_cus() * nt - 1) / ((int64_t)num_cus() * nt);
-  const int64_t per_group = (tiles + (int64_t)nt * passes - 1) / ((int64_t)nt * passes);
-  const int grid = (int)(groups * (per_group > 0 ? per_group : 1));
+  const GroupSpread sp = px3_spread<CO>(a);
+  const int grid = groups * sp.per_group, nt = sp.waves;
   constexpr auto kern = k_conv_px3<TIn, TOut, CO, LIF>;
   const int e = set_lds_limit_once<kern>(kMaxLdsBytes - 1024);
   if (e != (int)hipSuccess) return e;
@@ -1087,10 +1091,10 @@ int launch_px3_t(const ConvArgs& a, int out_dtype, hipStream_t stream) {
 }
 
 template <typename TIn, typename TOut, int CW>
-int launch_px3s_cw(const ConvArgs& a, int groups, int64_t tiles, int nt, hipStream_t stream, DenseQueue* dq) {
+int launch_px3s_cw(const ConvArgs& a, int groups, const GroupSpread& sp, hipStream_t stream, DenseQueue* dq) {
   typedef Px3Layout<64> LY;
   const int nchunks = (a.c_in + kPx3Ch - 1) / kPx3Ch;
-  const int grid = (int)(groups * ((tiles + nt - 1) / nt));
+  const int grid = groups * sp.per_group, nt = sp.waves;
   constexpr auto kern = k_conv_px3s<TIn, TOut, CW>;
   const int e = set_lds_limit_once<kern>(kMaxLdsBytes - 1024);
   if (e != (int)hipSuccess) return e;
@@ -1102,13 +1106,12 @@ int launch_px3s_cw(const ConvArgs& a, int groups, int64_t tiles, int nt, hipStre
 template <typename TIn, typename TOut>
 int launch_px3s_to(const ConvArgs& a, hipStream_t stream, DenseQueue** dense) {
   const int groups = (a.c_out + 63) / 64;
-  const int64_t tiles = (a.n * (int64_t)a.hw_out + 63) / 64;
-  const int nt = even_pass_waves(tiles * groups);
+  const GroupSpread sp = px3s_spread(a);
   // (Queue entries hold a run's first pixel of the flattened axis in 31 bits.)
   DenseQueue* dq =
       groups <= kDenseQueueGroups && a.n * (int64_t)a.hw_out < (1ll << 31) ? dense_queue_for(stream) : nullptr;
-  const int rc = nt <= kPx3SplitTiles ? launch_px3s_cw<TIn, TOut, 16>(a, groups, tiles, nt, stream, dq)
-                                       : launch_px3s_cw<TIn, TOut, 64>(a, groups, tiles, nt, stream, dq);
+  const int rc = sp.waves <= kPx3SplitTiles ? launch_px3s_cw<TIn, TOut, 16>(a, groups, sp, stream, dq)
+                                            : launch_px3s_cw<TIn, TOut, 64>(a, groups, sp, stream, dq);
   if (rc == (int)hipSuccess) *dense = dq;
   return rc;
 }
@@ -1120,62 +1123,64 @@ int launch_px3s_t(const ConvArgs& a, int out_dtype, hipStream_t stream, DenseQue
   return launch_px3s_to<TIn, float>(a, stream, dense);
 }
 
-template <int CO>
-int launch_px3_co(const ConvArgs& a, int in_dtype, int out_dtype, hipStream_t stream) {
-  if (in_dtype == SF_F16) return launch_px3_t<__half, float, CO, false>(a, out_dtype, stream);
-  if (in_dtype == SF_BF16) return launch_px3_t<__hip_bfloat16, float, CO, false>(a, out_dtype, stream);
-  return launch_px3_t<float, float, CO, false>(a, out_dtype, stream);
-}
-
 // Output channels per workgroup slice: 64, or 32 where that keeps the
 // weights resident in LDS (64 < C_in <= 128), which removes the per-pass
 // chunk streaming and its barriers at the cost of walking the spikes once
 // per slice.  (A 16-channel slice, resident up to C_in = 256, walks too
 // often: slower than streaming.)
-int launch_px3_conv(const ConvArgs& a, int in_dtype, int out_dtype, hipStream_t stream, DenseQueue** dense) {
+enum class Px3Form { kW64, kW32, kChunks32, kStreamed, kChunks64 };
+
+Px3Form px3_form(const ConvArgs& a, int out_dtype) {
   // C_in <= 64: one 64-channel super-chunk, every weight row resident, 64
   // output channels; 64 < C_in <= 128: 32-channel slices of all 128 input
   // channels' rows, two super-chunks.  (One sample's output planes must be
   // addressable by one buffer resource, with CO planes to spare.)
   const int out_bytes = out_dtype == SF_F32 ? 4 : 2;
   if ((int64_t)(a.c_out + 64) * a.hw_out * out_bytes < 0x7fffffffLL) {
-    if (a.c_in <= 64 && a.cwp <= 2) {
-      if (in_dtype == SF_F16) return launch_px3w_t<__half, 64>(a, out_dtype, stream);
-      if (in_dtype == SF_BF16) return launch_px3w_t<__hip_bfloat16, 64>(a, out_dtype, stream);
-      return launch_px3w_t<float, 64>(a, out_dtype, stream);
-    }
-    if (a.c_in <= 128 && a.cwp <= 4) {
-      if (in_dtype == SF_F16) return launch_px3w_t<__half, 32>(a, out_dtype, stream);
-      if (in_dtype == SF_BF16) return launch_px3w_t<__hip_bfloat16, 32>(a, out_dtype, stream);
-      return launch_px3w_t<float, 32>(a, out_dtype, stream);
-    }
+    if (a.c_in <= 64 && a.cwp <= 2) return Px3Form::kW64;
+    if (a.c_in <= 128 && a.cwp <= 4) return Px3Form::kW32;
   }
   const int nch = (a.c_in + kPx3Ch - 1) / kPx3Ch;
-  if (nch > Px3Layout<64>::resident_chunks && nch <= Px3Layout<32>::resident_chunks)
-    return launch_px3_co<32>(a, in_dtype, out_dtype, stream);
+  if (nch > Px3Layout<64>::resident_chunks && nch <= Px3Layout<32>::resident_chunks) return Px3Form::kChunks32;
   // C_in > 128: streamed chunks over flattened tiles, when every frame's
   // bitmap and every frame's output planes are addressable by one buffer
   // resource each.
   if (nch > Px3Layout<32>::resident_chunks && a.n * (int64_t)a.hw_in * a.cwp * 4 < 0x7fffffffLL &&
-      a.n * (int64_t)(a.c_out + 64) * a.hw_out * out_bytes < 0x7fffffffLL) {
-    if (in_dtype == SF_F16) return launch_px3s_t<__half>(a, out_dtype, stream, dense);
-    if (in_dtype == SF_BF16) return launch_px3s_t<__hip_bfloat16>(a, out_dtype, stream, dense);
-    return launch_px3s_t<float>(a, out_dtype, stream, dense);
+      a.n * (int64_t)(a.c_out + 64) * a.hw_out * out_bytes < 0x7fffffffLL)
+    return Px3Form::kStreamed;
+  return Px3Form::kChunks64;
+}
+
+template <typename TIn>
+int launch_px3_conv_t(const ConvArgs& a, int out_dtype, hipStream_t stream, DenseQueue** dense) {
+  switch (px3_form(a, out_dtype)) {
+    case Px3Form::kW64: return launch_px3w_t<TIn, 64>(a, out_dtype, stream);
+    case Px3Form::kW32: return launch_px3w_t<TIn, 32>(a, out_dtype, stream);
+    case Px3Form::kChunks32: return launch_px3_t<TIn, float, 32, false>(a, out_dtype, stream);
+    case Px3Form::kStreamed: return launch_px3s_t<TIn>(a, out_dtype, stream, dense);
+    default: return launch_px3_t<TIn, float, 64, false>(a, out_dtype, stream);
   }
-  return launch_px3_co<64>(a, in_dtype, out_dtype, stream);
+}
+
+int launch_px3_conv(const ConvArgs& a, int in_dtype, int out_dtype, hipStream_t stream, DenseQueue** dense) {
+  if (in_dtype == SF_F16) return launch_px3_conv_t<__half>(a, out_dtype, stream, dense);
+  if (in_dtype == SF_BF16) return launch_px3_conv_t<__hip_bfloat16>(a, out_dtype, stream, dense);
+  return launch_px3_conv_t<float>(a, out_dtype, stream, dense);
 }
 
 // Fused LIF: 32 output channels per workgroup.  The membrane shares the
 // accumulator registers, and with 32 channels the weights of up to 128 input
 // channels stay resident (config 4) and a sample's tiles spread over twice
 // as many workgroups.
+bool lif_resident(const ConvArgs& a) { return a.c_in <= 128 && a.cwp <= 4; }
+
 template <typename TIn, typename TOut>
 int launch_px3_lif_t(const ConvArgs& a, hipStream_t stream) {
   // Up to 128 input channels: every weight row resident and the spikes
   // walked as 64-channel super-chunks (fewer rounds than 32-channel chunks:
   // a round count is the busiest lane's, which grows more slowly than the
   // mean).
-  if (a.c_in <= 128 && a.cwp <= 4) return launch_px3w_to<TIn, TOut, 32, true>(a, stream);
+  if (lif_resident(a)) return launch_px3w_to<TIn, TOut, 32, true>(a, stream);
   return launch_px3_t<TIn, TOut, 32, true>(a, 0, stream);
 }
 
@@ -1202,6 +1207,14 @@ bool px3_applicable(const ConvArgs& a) {
   // 2^31.)
   return a.k == 3 && a.p == 1 && (a.s == 1 || a.s == 2) && a.c_out % 4 == 0 && a.cwp <= 64 &&
          a.n * (int64_t)((a.hw_out + 63) / 64) < (1ll << 30) && (int64_t)a.hw_in * a.cwp * 4 < (1ll << 31);
+}
+
+LaunchPlan px3_plan(const ConvArgs& a, int out_dtype, bool lif) {
+  const Px3Form form = lif ? (lif_resident(a) ? Px3Form::kW32 : Px3Form::kChunks32) : px3_form(a, out_dtype);
+  const int co = form == Px3Form::kW32 || form == Px3Form::kChunks32 ? 32 : 64;
+  const GroupSpread sp = form == Px3Form::kStreamed ? px3s_spread(a) : co == 32 ? px3_spread<32>(a) : px3_spread<64>(a);
+  const bool split = form != Px3Form::kChunks32 && form != Px3Form::kChunks64 && sp.waves <= kPx3SplitTiles;
+  return {(a.c_out + co - 1) / co * sp.per_group, sp.waves, split ? 4 : 1};
 }
 
 int launch_conv_px3(const ConvArgs& a, int in_dtype, int out_dtype, hipStream_t stream) {

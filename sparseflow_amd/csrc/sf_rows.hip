@@ -282,20 +282,24 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_rows_kc(ConvArgs a, co
   }
 }
 
+// (w_out is 28 or 14)
+GroupSpread kc_spread(const ConvArgs& a) {
+  const int th = a.w_out == 28 ? 2 : 4;
+  const int64_t tiles = a.n * (int64_t)((a.h_out + th - 1) / th);
+  // As many tiles per workgroup as spread them evenly over the CUs: full
+  // workgroups of 16 leave most CUs idle at small batches (us, 4 / 16 / 64 x 256
+  // x 14 x 14 -> 256: 49.7 -> 37.7, 51.2 -> 39.3, 53.1 -> 43.8; 16 x 256 x 28 x 28 ->
+  // 256 60.2 -> 50.4; 512 x 256 x 14 x 14 -> 256, full either way, 106.6 / 104.5).
+  return spread_passes(tiles, (a.c_out + 63) / 64);
+}
+
 template <int TH, int W>
 int launch_kc_t(const ConvArgs& a, int in_dtype, int out_dtype, hipStream_t stream, DenseQueue** dense) {
   const int groups = (a.c_out + 63) / 64;
   const int nchunks = (a.c_in + 31) / 32;
   const size_t lds = (size_t)2 * kChunkBytes;
-  const int64_t tiles = a.n * (int64_t)((a.h_out + TH - 1) / TH);
-  // As many tiles per workgroup as spread them evenly over the CUs: full
-  // workgroups of 16 leave most CUs idle at small batches (us, 4 / 16 / 64 x 256
-  // x 14 x 14 -> 256: 49.7 -> 37.7, 51.2 -> 39.3, 53.1 -> 43.8; 16 x 256 x 28 x 28 ->
-  // 256 60.2 -> 50.4; 512 x 256 x 14 x 14 -> 256, full either way, 106.6 / 104.5).
-  const int nt = even_pass_waves(tiles * groups);
-  const int64_t passes = (tiles * groups + (int64_t)num_cus() * nt - 1) / ((int64_t)num_cus() * nt);
-  const int64_t per_group = (tiles + (int64_t)nt * passes - 1) / ((int64_t)nt * passes);
-  const int grid = (int)(groups * (per_group > 0 ? per_group : 1));
+  const GroupSpread sp = kc_spread(a);
+  const int grid = groups * sp.per_group, nt = sp.waves;
   constexpr auto kern = k_conv_rows_kc<TH, W>;
   const int e = set_lds_limit_once<kern>(kMaxLdsBytes);
   if (e != (int)hipSuccess) return e;
@@ -330,6 +334,11 @@ bool rows_kc_applicable(const ConvArgs& a) {
   return a.k == 3 && a.s == 1 && a.p == 1 && a.h_out == a.h_in && a.w_out == a.w_in &&
          (a.w_out == 28 || a.w_out == 14) && a.c_out % 4 == 0 && a.hw_out % 4 == 0 &&
          a.n * (int64_t)a.h_out < (1ll << 30);
+}
+
+LaunchPlan rows_kc_plan(const ConvArgs& a) {
+  const GroupSpread sp = kc_spread(a);
+  return {(a.c_out + 63) / 64 * sp.per_group, sp.waves, 1};
 }
 
 int launch_conv_rows_kc(const ConvArgs& a, int in_dtype, int out_dtype, hipStream_t stream) {

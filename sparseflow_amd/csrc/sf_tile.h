@@ -22,6 +22,39 @@ inline int even_pass_waves(int64_t wave_tiles) {
   return (int)(w < 1 ? 1 : (w > kRowsWaves ? kRowsWaves : w));
 }
 
+// How the wave-tiles of a layer are dealt out where every channel group has
+// workgroups of its own and one workgroup fills a CU's LDS: `waves` tiles a
+// pass for each of `per_group` workgroups a group.
+struct GroupSpread {
+  int waves;
+  int per_group;
+};
+
+// For workgroups that stay and make passes (resident weights): all of them on
+// the chip at once, the passes that 16 tiles each would need, and no more tiles
+// a pass than those take.  The groups are rounded one by one: counted over all
+// tiles together (even_pass_waves), a few workgroups could be left over for a
+// second round of the whole chip (32 x 256 x 14 x 14 -> 384, six groups of 128
+// tiles: 3 tiles each were 258 workgroups, 78 us; 4 are 192).
+inline GroupSpread spread_passes(int64_t tiles, int64_t groups) {
+  const int64_t slots = num_cus() > groups ? num_cus() / groups : 1;
+  const int64_t passes = tiles > 0 ? (tiles + slots * kRowsWaves - 1) / (slots * kRowsWaves) : 1;
+  const int64_t waves = tiles > 0 ? (tiles + slots * passes - 1) / (slots * passes) : 1;
+  const int64_t per_group = tiles > 0 ? (tiles + waves * passes - 1) / (waves * passes) : 1;
+  return {(int)waves, (int)per_group};
+}
+
+// For workgroups of one pass each, taken by the CUs as these come free: as many
+// rounds of the chip as 16 tiles each would need, and no more tiles than those
+// rounds take.
+inline GroupSpread spread_rounds(int64_t tiles, int64_t groups) {
+  const int64_t cus = num_cus();
+  const int64_t full = tiles > 0 ? (tiles + kRowsWaves - 1) / kRowsWaves : 1;
+  const int64_t slots = (groups * full + cus - 1) / cus * cus / groups;  // a group's workgroups in all rounds
+  const int64_t waves = tiles > 0 ? (tiles + slots - 1) / slots : 1;
+  return {(int)waves, (int)(tiles > 0 ? (tiles + waves - 1) / waves : 1)};
+}
+
 namespace {
 
 // Exchange lane bit S with quad-slot bit S over v[4 * QP] (a butterfly stage

@@ -258,3 +258,48 @@ def test_layout_requests_pick_planes_only_when_every_consumer_asks():
     assert r.layout == PLANES and len(r._wants) == LayoutRequests._MAX
     r.clear()
     assert r.layout == PIXEL_MAJOR
+
+
+# ---- launch plans of the tile kernels ----------------------------------------
+
+CUS = 256  # of the MI355X; assumed where there is no GPU
+
+
+def _plan(n, c_in, h, w, c_out, s=1, lif=False):
+    ho, wo = -(-h // s), -(-w // s)
+    d = _lib.conv_desc(n, c_in, h, w, c_out, ho, wo, 3, s, 1, _lib.SF_F32, _lib.SF_F32)
+    return _lib.conv2d_launch_plan(d, lif)
+
+
+# One workgroup fills a CU's LDS, so workgroups past the CUs wait for a second
+# round.  Wherever workgroups of 16 tiles fit the chip at once, the spread ones
+# do too, and one tile less would not have fitted.
+@pytest.mark.parametrize("c_in,size,lif", [(256, 14, False), (192, 28, False), (256, 8, False), (130, 17, False),
+                                           (100, 16, False), (64, 20, False), (256, 14, True), (150, 28, True),
+                                           (128, 14, True), (40, 28, True)])
+def test_tiles_spread_within_one_round_of_cus(c_in, size, lif):
+    rows = not lif and c_in > 128 and size in (14, 28)          # four- and two-row tiles
+    streamed = not lif and c_in > 128 and not rows               # 64-pixel tiles over all frames
+    co_group = 32 if lif or 64 < c_in <= 128 else 64
+    for groups in list(range(1, 25)) + [40, 64]:
+        for n in (1, 2, 3, 5, 8, 10, 16, 19, 32, 37, 48, 64, 96, 100, 128, 200, 256, 320):
+            wg, nt, _ = _plan(n, c_in, size, size, groups * co_group, lif=lif)
+            px = size * size
+            tiles = n * (size // 2 if size == 28 else -(-size // 4)) if rows else \
+                -(-n * px // 64) if streamed else n * -(-px // 64)
+            assert 1 <= nt <= 16 and wg % groups == 0
+            if groups * -(-tiles // 16) <= CUS:
+                assert wg <= CUS, (n, groups)
+                assert nt * (wg // groups) >= tiles, (n, groups)
+                assert nt == 1 or groups * -(-tiles // (nt - 1)) > CUS, (n, groups)
+
+
+def test_launch_plan_known_shapes():
+    # six groups of 128 four-row tiles: three tiles each would be 6 x 43 = 258 workgroups
+    assert _plan(32, 256, 14, 14, 384) == (6 * 32, 4, 1)
+    assert _plan(128, 256, 14, 14, 192) == (3 * 74, 7, 1)
+    assert _plan(16, 256, 14, 14, 384, lif=True) == (12 * 16, 4, 1)
+    # other kernels have no such plan
+    d = _lib.conv_desc(4, 64, 8, 8, 64, 8, 8, 1, 1, 0, 0, 0)
+    with pytest.raises(_lib.UnsupportedError):
+        _lib.conv2d_launch_plan(d)
