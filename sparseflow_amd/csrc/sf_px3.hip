@@ -1031,15 +1031,20 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3w(ConvArgs a, const
   }
 }
 
-// Frame by frame in 64-pixel tiles (px3, px3w), CO channels to a group.
+// Frame by frame in 64-pixel tiles, CO channels to a group: px3w's workgroups,
+// whose weights stay in LDS, make passes.
+template <int CO>
+GroupSpread px3w_spread(const ConvArgs& a) {
+  return spread_passes(a.n * (int64_t)((a.hw_out + 63) / 64), (a.c_out + CO - 1) / CO);
+}
 template <int CO>
 GroupSpread px3_spread(const ConvArgs& a) {
-  return spread_passes(a.n * (int64_t)((a.hw_out + 63) / 64), (a.c_out + CO - 1) / CO);
+  return spread_rounds(a.n * (int64_t)((a.hw_out + 63) / 64), (a.c_out + CO - 1) / CO, 2);
 }
 
 // Over the flattened (frame, pixel) axis (px3s).
 GroupSpread px3s_spread(const ConvArgs& a) {
-  return spread_rounds((a.n * (int64_t)a.hw_out + 63) / 64, (a.c_out + 63) / 64);
+  return spread_rounds((a.n * (int64_t)a.hw_out + 63) / 64, (a.c_out + 63) / 64, INT64_MAX);
 }
 
 template <typename TIn, typename TOut, int CO, bool LIF, int CW>
@@ -1057,7 +1062,7 @@ int launch_px3w_to(const ConvArgs& a, hipStream_t stream) {
   const int groups = (a.c_out + CO - 1) / CO;
   // One workgroup per CU (the weights fill the LDS) making the same number
   // of passes: no CU idles through another's last pass.
-  const GroupSpread sp = px3_spread<CO>(a);
+  const GroupSpread sp = px3w_spread<CO>(a);
   const int grid = groups * sp.per_group, nt = sp.waves;
   return nt <= kPx3SplitTiles ? launch_px3w_cw<TIn, TOut, CO, LIF, CO / 4>(a, grid, groups, nt, stream)
                               : launch_px3w_cw<TIn, TOut, CO, LIF, CO>(a, grid, groups, nt, stream);
@@ -1077,8 +1082,8 @@ int launch_px3_t(const ConvArgs& a, int out_dtype, hipStream_t stream) {
   const int nchunks = (a.c_in + kPx3Ch - 1) / kPx3Ch;
   const int held = nchunks <= LY::resident_chunks ? nchunks : 2;
   const size_t lds = (size_t)held * LY::chunk_bytes;
-  // The tiles spread over the CUs as in launch_px3w_to: full workgroups of 16
-  // left most of them idle (fused LIF, 4 x 8 x 200 x 14 x 14 -> 200: 173 -> 117
+  // The tiles spread over the CUs: full workgroups of 16 left most of them
+  // idle (fused LIF, 4 x 8 x 200 x 14 x 14 -> 200: 173 -> 117
   // us).
   const GroupSpread sp = px3_spread<CO>(a);
   const int grid = groups * sp.per_group, nt = sp.waves;
@@ -1212,7 +1217,14 @@ bool px3_applicable(const ConvArgs& a) {
 LaunchPlan px3_plan(const ConvArgs& a, int out_dtype, bool lif) {
   const Px3Form form = lif ? (lif_resident(a) ? Px3Form::kW32 : Px3Form::kChunks32) : px3_form(a, out_dtype);
   const int co = form == Px3Form::kW32 || form == Px3Form::kChunks32 ? 32 : 64;
-  const GroupSpread sp = form == Px3Form::kStreamed ? px3s_spread(a) : co == 32 ? px3_spread<32>(a) : px3_spread<64>(a);
+  GroupSpread sp;
+  switch (form) {
+    case Px3Form::kW64: sp = px3w_spread<64>(a); break;
+    case Px3Form::kW32: sp = px3w_spread<32>(a); break;
+    case Px3Form::kStreamed: sp = px3s_spread(a); break;
+    case Px3Form::kChunks32: sp = px3_spread<32>(a); break;
+    default: sp = px3_spread<64>(a);
+  }
   const bool split = form != Px3Form::kChunks32 && form != Px3Form::kChunks64 && sp.waves <= kPx3SplitTiles;
   return {(a.c_out + co - 1) / co * sp.per_group, sp.waves, split ? 4 : 1};
 }

@@ -290,7 +290,9 @@ GroupSpread kc_spread(const ConvArgs& a) {
   // workgroups of 16 leave most CUs idle at small batches (us, 4 / 16 / 64 x 256
   // x 14 x 14 -> 256: 49.7 -> 37.7, 51.2 -> 39.3, 53.1 -> 43.8; 16 x 256 x 28 x 28 ->
   // 256 60.2 -> 50.4; 512 x 256 x 14 x 14 -> 256, full either way, 106.6 / 104.5).
-  return spread_passes(tiles, (a.c_out + 63) / 64);
+  // Past two rounds the last one's share is small, and full workgroups spread a
+  // burst over fewer CUs (90 x 256 x 28 x 28 -> 512, bursts: 201 even, 191 full).
+  return spread_rounds(tiles, (a.c_out + 63) / 64, 2);
 }
 
 template <int TH, int W>

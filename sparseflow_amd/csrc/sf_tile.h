@@ -37,22 +37,29 @@ struct GroupSpread {
 // second round of the whole chip (32 x 256 x 14 x 14 -> 384, six groups of 128
 // tiles: 3 tiles each were 258 workgroups, 78 us; 4 are 192).
 inline GroupSpread spread_passes(int64_t tiles, int64_t groups) {
+  if (tiles < 1) return {1, 1};
   const int64_t slots = num_cus() > groups ? num_cus() / groups : 1;
-  const int64_t passes = tiles > 0 ? (tiles + slots * kRowsWaves - 1) / (slots * kRowsWaves) : 1;
-  const int64_t waves = tiles > 0 ? (tiles + slots * passes - 1) / (slots * passes) : 1;
-  const int64_t per_group = tiles > 0 ? (tiles + waves * passes - 1) / (waves * passes) : 1;
-  return {(int)waves, (int)per_group};
+  const int64_t passes = (tiles + slots * kRowsWaves - 1) / (slots * kRowsWaves);
+  const int64_t waves = (tiles + slots * passes - 1) / (slots * passes);
+  return {(int)waves, (int)((tiles + waves * passes - 1) / (waves * passes))};
 }
 
 // For workgroups of one pass each, taken by the CUs as these come free: as many
-// rounds of the chip as 16 tiles each would need, and no more tiles than those
-// rounds take.
-inline GroupSpread spread_rounds(int64_t tiles, int64_t groups) {
+// rounds of the chip as 16 tiles each would need and, up to `even` rounds, no
+// more tiles than those rounds take.  Where the weights are streamed anyway,
+// this beats workgroups that stay: a live network's spikes come in bursts of a
+// few frames, and a CU whose workgroup met one would keep its share of the rest
+// (us, passes -> rounds, one time step of 16 at ten times the mean density and
+// one at 3.2 times, row kernel: 512 x 256 x 14 x 14 -> 256 183 -> 157, 256 x 256
+// x 28 x 28 -> 128 203 -> 175, 512 x 512 x 14 x 14 -> 512 465 -> 415; evenly
+// spread spikes, the first: 118 -> 121).
+inline GroupSpread spread_rounds(int64_t tiles, int64_t groups, int64_t even) {
+  if (tiles < 1) return {1, 1};
   const int64_t cus = num_cus();
-  const int64_t full = tiles > 0 ? (tiles + kRowsWaves - 1) / kRowsWaves : 1;
-  const int64_t slots = (groups * full + cus - 1) / cus * cus / groups;  // a group's workgroups in all rounds
-  const int64_t waves = tiles > 0 ? (tiles + slots - 1) / slots : 1;
-  return {(int)waves, (int)(tiles > 0 ? (tiles + waves - 1) / waves : 1)};
+  const int64_t rounds = (groups * ((tiles + kRowsWaves - 1) / kRowsWaves) + cus - 1) / cus;
+  const int64_t slots = rounds * cus / groups;  // a group's workgroups in all rounds
+  const int64_t waves = rounds <= even ? (tiles + slots - 1) / slots : kRowsWaves;
+  return {(int)waves, (int)((tiles + waves - 1) / waves)};
 }
 
 namespace {

@@ -294,6 +294,23 @@ def test_tiles_spread_within_one_round_of_cus(c_in, size, lif):
                 assert nt == 1 or groups * -(-tiles // (nt - 1)) > CUS, (n, groups)
 
 
+# The kernels that stream their weights give every pass a workgroup of its own
+# (spikes that come in bursts keep a workgroup for long: the CUs take the others
+# as they come free); those with resident weights make passes.
+def test_streamed_tiles_take_a_workgroup_per_pass():
+    for n, groups in ((512, 4), (300, 4), (512, 8), (1024, 4), (2000, 1)):
+        wg, nt, _ = _plan(n, 256, 14, 14, 64 * groups)                  # row tiles
+        assert nt * (wg // groups) >= 4 * n > nt * (wg // groups - 1)
+        wg, nt, _ = _plan(n, 256, 14, 14, 32 * groups, lif=True)        # fused LIF
+        assert nt * (wg // groups) >= 4 * n > nt * (wg // groups - 1)
+        wg, nt, _ = _plan(n, 256, 16, 16, 64 * groups)                  # flattened tiles
+        assert nt * (wg // groups) >= 4 * n > nt * (wg // groups - 1)
+        wg, nt, _ = _plan(n, 128, 16, 16, 32 * groups)                  # resident
+        assert wg <= CUS
+    assert _plan(300, 256, 14, 14, 256) == (4 * 120, 10, 1)             # two rounds, evenly
+    assert _plan(90, 256, 28, 28, 512) == (8 * 79, 16, 1)               # three: full workgroups
+
+
 def test_launch_plan_known_shapes():
     # six groups of 128 four-row tiles: three tiles each would be 6 x 43 = 258 workgroups
     assert _plan(32, 256, 14, 14, 384) == (6 * 32, 4, 1)
