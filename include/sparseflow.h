@@ -375,6 +375,15 @@ int sf_linear_mfma_bits(const uint32_t* bits, const uint32_t* flags,
                         const float* bias, int32_t c_out, float threshold,
                         void* y, int32_t out_dtype, void* stream);
 
+/* Host only, for the shapes above (of x only the alignment is looked at):
+ * sf_linear_mfma's tiles -- 4, 8 or 13 for workgroups of 16 times as many rows
+ * x 384 columns, 0 for 128 x 128 -- and whether prescan + sf_linear_mfma_bits
+ * is expected to be the faster way. */
+int sf_linear_mfma_row_tiles(const void* x, int32_t in_dtype, int64_t m,
+                             int32_t k, int32_t c_out);
+int sf_linear_mfma_bits_pays(const void* x, int32_t in_dtype, int64_t m,
+                             int32_t k, int32_t c_out);
+
 /* ---- sparse batched matmul -------------------------------------------------- */
 
 /* c[b] = alpha * (a[b] @ B[b]) for b < batches: a [batches, m, k] contiguous and

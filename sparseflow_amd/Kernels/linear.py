@@ -14,13 +14,14 @@
                              with the A operand of spike row blocks from the
                              bitmap (flagged blocks read x, split the same
                              way); the row prescan (one read of x) pays off
-                             when a wide output is large: see
-                             `_bitmap_pays`
+                             where `linear_mfma_bits_pays` says so: wide
+                             outputs that are large or that the direct kernel
+                             does not clearly do faster
 
 The walk does ~density x the MACs on the VALU; the MFMA tile paths do them
 all on the matrix cores and win once every 32-wide K slice of a 128-row tile
 is live (transformer densities, p ~ 0.1).  `kernel="auto"` takes the walk
-for k < 32, "mfma_bits" where `_bitmap_pays` says so and "mfma" otherwise;
+for k < 32, "mfma_bits" where the bitmap pays off and "mfma" otherwise;
 on binary x both give the same bits.
 
 Weights stay fp32 and the sum is fp32 (the reference casts x and W to fp16
@@ -52,37 +53,6 @@ def _select_linear_block_m(n_rows: int) -> int:
     if n_rows >= 256:
         return 64
     return 32
-
-
-def _bitmap_pays(x: torch.Tensor, n: int, k: int, c_out: int) -> bool:
-    """Whether the row bitmap and "mfma_bits" beat "mfma" on x [n, k].
-
-    Only outputs at least twice as wide as the input reuse the bitmap enough,
-    and only large ones repay its launch (us, bitmap / direct, 10% spikes):
-
-      f32   50176 x 384 -> 1536  153 / 165    32768 x 512 -> 2048  146 / 184
-            65536 x 192 -> 768   63 / 71      8192 x 768 -> 3072   98 / 85
-            25088 x 384 -> 1536  81 / 71      8192 x 512 -> 2048   50 / 46
-            4096 x 1024 -> 4096  81 / 73      1000 x 384 -> 1536   29 / 15
-            65536 x 128 -> 512   42 / 36      10000 x 64 -> 256    16 / 7
-      f16   50176 x 384 -> 1536  158 / 157    8192 x 512 -> 2048   80 / 50
-            65536 x 192 -> 768   72 / 79      8192 x 768 -> 3072   153 / 89
-            65536 x 128 -> 512   42 / 52      32768 x 128 -> 512   31 / 28
-            100000 x 64 -> 256   30 / 34      50000 x 64 -> 256    20 / 19
-      f32, k no multiple of 16 or x off 16 bytes (single-element loads in
-      the direct kernel for k < 192)
-            50176 x 385 -> 1536  172 / 216    8192 x 514 -> 2048   63 / 55
-            65536 x 129 -> 512   49 / 65      30000 x 161 -> 640   41 / 38
-
-    x of full precision is faster direct throughout (50176 x 384 -> 1536
-    408 / 239).
-    """
-    if c_out < 2 * k:
-        return False
-    if k < 192:
-        wide_loads = x.dtype == torch.float32 and k % 16 == 0 and x.data_ptr() % 16 == 0
-        return not wide_loads and n * c_out >= 25_000_000
-    return n * c_out >= 45_000_000
 
 
 def unpack_row_bits(bits: torch.Tensor, m: int, k: int) -> torch.Tensor:
@@ -212,7 +182,9 @@ def sparse_linear_forward(
     x = x.contiguous()
     lib_out = out_dtype if out_dtype in (x.dtype, torch.float32) else torch.float32
     use_mfma = kernel in ("mfma", "mfma_bits") or (kernel == "auto" and C_IN >= 32)
-    mfma_bits = kernel == "mfma_bits" or (kernel == "auto" and C_IN >= 32 and _bitmap_pays(x, N, C_IN, C_OUT))
+    mfma_bits = kernel == "mfma_bits" or (
+        kernel == "auto" and C_IN >= 32 and C_OUT >= 2 * C_IN
+        and _lib.linear_mfma_bits_pays(N, C_IN, C_OUT, x.dtype, x.data_ptr() % 16))
     wt = None
     if not use_mfma:
         if w_t is not None and tuple(w_t.shape) == (C_IN, C_OUT):

@@ -11,6 +11,7 @@ SparseFlowLibError: there is no silent fallback for ROCm tensors.
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from ctypes import c_double, c_float, c_int, c_int32, c_int64, c_size_t, c_uint32, c_void_p
 from pathlib import Path
@@ -74,6 +75,8 @@ EXPORTS = {
                                   _P]),
     "sf_linear_mfma": (c_int, [_P, c_int32, c_int64, c_int32, _P, _P, c_int32, _P, c_int32, c_float, _P, c_int32,
                                _P]),
+    "sf_linear_mfma_row_tiles": (c_int, [_P, c_int32, c_int64, c_int32, c_int32]),
+    "sf_linear_mfma_bits_pays": (c_int, [_P, c_int32, c_int64, c_int32, c_int32]),
     "sf_linear_mfma_bits": (c_int, [_P, _P, _P, c_int32, c_int64, c_int32, _P, _P, c_int32, _P, c_int32, c_float, _P,
                                     c_int32, _P]),
     "sf_bmm_supported": (c_int, [c_int32, c_int32]),
@@ -490,6 +493,20 @@ def linear_mfma(x2d: torch.Tensor, w_hi: torch.Tensor, w_lo: torch.Tensor, bias:
                               float(threshold), _ptr(y), dtype_code(y.dtype), _stream(x2d.device))
     _check(rc, "sf_linear_mfma")
     return y
+
+
+@functools.lru_cache(maxsize=1024)
+def linear_mfma_row_tiles(m: int, k: int, c_out: int, dtype: torch.dtype, offset: int = 0) -> int:
+    """16-row tiles of linear_mfma's 384-column workgroups, 0 where it runs
+    128 x 128 tiles (sf_linear_mfma_row_tiles); offset: x's address modulo 16."""
+    return int(lib().sf_linear_mfma_row_tiles(offset, dtype_code(dtype), m, k, c_out))
+
+
+@functools.lru_cache(maxsize=1024)
+def linear_mfma_bits_pays(m: int, k: int, c_out: int, dtype: torch.dtype, offset: int = 0) -> bool:
+    """Whether linear_prescan + linear_mfma_bits are expected to be faster than
+    linear_mfma (sf_linear_mfma_bits_pays); offset: x's address modulo 16."""
+    return bool(lib().sf_linear_mfma_bits_pays(offset, dtype_code(dtype), m, k, c_out))
 
 
 def linear_mfma_bits(bits: torch.Tensor, flags: torch.Tensor, x2d: torch.Tensor, w_hi: torch.Tensor,

@@ -564,6 +564,16 @@ int sf_linear_mfma(const void* x, int32_t in_dtype, int64_t m, int32_t k, const 
   return SF_OK;
 }
 
+int sf_linear_mfma_row_tiles(const void* x, int32_t in_dtype, int64_t m, int32_t k, int32_t c_out) {
+  if (m < 1 || k < 1 || c_out < 1 || !dtype_ok(in_dtype)) return 0;
+  return sf::linear_mfma_row_tiles(x, in_dtype, m, k, c_out);
+}
+
+int sf_linear_mfma_bits_pays(const void* x, int32_t in_dtype, int64_t m, int32_t k, int32_t c_out) {
+  if (m < 1 || k < 1 || c_out < 1 || !dtype_ok(in_dtype)) return 0;
+  return sf::linear_mfma_bits_pays(x, in_dtype, m, k, c_out) ? 1 : 0;
+}
+
 int sf_linear_mfma_bits(const uint32_t* bits, const uint32_t* flags, const void* x, int32_t in_dtype, int64_t m,
                         int32_t k, const uint16_t* w_hi, const uint16_t* w_lo, int32_t kp, const float* bias,
                         int32_t c_out, float threshold, void* y, int32_t out_dtype, void* stream) {

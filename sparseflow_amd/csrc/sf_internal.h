@@ -239,6 +239,10 @@ struct LinMfmaArgs {
   float cutoff;  // elements with |x| < cutoff count as zero
 };
 int linear_mfma_max_kp();
+// 16-row tiles of a workgroup of the 384-column kernel, or 0 where
+// launch_linear_mfma runs 128 x 128 tiles (of x only the alignment counts).
+int linear_mfma_row_tiles(const void* x, int in_dtype, int64_t m, int k, int c_out);
+bool linear_mfma_bits_pays(const void* x, int in_dtype, int64_t m, int k, int c_out);
 int launch_linear_mfma(const LinMfmaArgs& a, int in_dtype, int out_dtype, hipStream_t stream);
 // The same product over sf_linear_prescan's row bitmap (cwp words per row)
 // and its non-binary flags (one per kLinearRowChunk rows).

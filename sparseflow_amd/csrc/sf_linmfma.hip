@@ -30,6 +30,8 @@
 // Replaces the reference's sparse_linear_grouped_kernel (Kernels/linear.py:
 // 360-457: fp16 tl.dot over active groups, dense tiles when all groups are
 // live) for such inputs.
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "sf_tile.h"
@@ -834,6 +836,59 @@ bool lm_vec(const LinMfmaArgs& a) {  // k_linear_mfma's 16-byte loads
   return sizeof(TIn) == 4 && a.k % 16 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0;
 }
 
+// What the choice of a kernel looks at.
+struct LinShape {
+  int64_t m;
+  int k, c_out, e;  // e: bytes of an element of x
+  bool vec;         // k_linear_mfma's 16-byte loads
+  int cus;
+};
+
+LinShape lin_shape(int64_t m, int k, int c_out, int in_dtype, const void* x) {
+  const bool f32 = in_dtype == SF_F32;
+  return {m, k, c_out, f32 ? 4 : 2, f32 && k % 16 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0,
+          num_cus()};
+}
+
+// Estimated times of the three kernels (us): per K step and workgroup of a CU
+// (per round of workgroups for k_linear_wide), and per MB of y and of x.
+// Fitted to 7,000 shapes of k 32 to 2048, c_out 16 to 2048 and up to 131,072
+// rows, binary x, inputs and outputs changing from call to call; nine in ten
+// estimates are within 15% (short k with a wide y is overestimated, by up to
+// a half).
+double lin_mb(const LinShape& s, int cols) { return 1e-6 * (double)s.m * cols * s.e; }
+int64_t lin_blocks(int64_t n, int64_t per) { return (n + per - 1) / per; }
+double lin_per_cu(const LinShape& s, int64_t workgroups) { return (double)lin_blocks(workgroups, s.cus); }
+
+double lm_us(const LinShape& s) {
+  const double steps = (double)lin_blocks(s.k, kLmK), y = lin_mb(s, s.c_out), x = lin_mb(s, s.k);
+  const double n = lin_per_cu(s, lin_blocks(s.m, kLmRows) * lin_blocks(s.c_out, kLmCols)), n3 = std::ceil(n / 3);
+  // Single elements loaded from rows of whole 64-byte lines: every lane's in
+  // the same place of its line, a quarter slower.
+  const bool in_step = s.k * s.e % 64 == 0;
+  if (s.vec) return 2.8 + steps * (0.8 * n3 + 0.32 * n) + 0.197 * y + 0.087 * x;
+  if (s.e == 4 && in_step) return 4.0 + steps * (0.47 * n3 + 1.8 * n) + 0.167 * y + 0.07 * x;
+  if (s.e == 4) return 2.6 + steps * (0.48 * n3 + 1.44 * n) + 0.122 * y + 0.167 * x;
+  if (in_step) return 3.9 + steps * (0.7 * n3 + 1.84 * n) + 0.244 * y + 0.053 * x;
+  return 2.6 + steps * (0.61 * n3 + 1.32 * n) + 0.158 * y + 0.142 * x;
+}
+
+double lw_us(const LinShape& s, int rt) {
+  const double steps = (double)lin_blocks(s.k, kLmK), y = lin_mb(s, s.c_out), x = lin_mb(s, s.k);
+  const double rounds = lin_per_cu(s, lin_blocks(s.m, 16 * rt) * lin_blocks(s.c_out, kLwCols));
+  if (s.e == 4)  // (a store writes 64 bytes of a row: whole lines where the rows of y start on them)
+    return 0.6 + rounds * (4.0 + steps * (0.29 + 0.12 * rt)) + (s.c_out % 16 != 0 ? 0.404 : 0.244) * y + 0.06 * x;
+  return 0.5 + rounds * (4.3 + steps * (0.21 + 0.138 * rt)) + 0.46 * y + 0.042 * x;
+}
+
+double lb_us(const LinShape& s) {  // with the row prescan
+  const double steps = (double)lin_blocks(s.k, kLmK), y = lin_mb(s, s.c_out), x = lin_mb(s, s.k);
+  const double n = lin_per_cu(s, lin_blocks(s.m, kLbRows) * lin_blocks(s.c_out, kLmCols));
+  if (s.vec) return 10.8 + 0.57 * n + steps * (0.58 + 0.62 * n) + 0.128 * y + 0.177 * x;
+  if (s.e == 4) return 8.2 + 1.9 * n + steps * (1.03 + 0.65 * n) + 0.085 * y + 0.16 * x;
+  return 7.9 + steps * (2.12 + 0.79 * n) + 0.195 * y + 0.78 * x;
+}
+
 // The number of 16-row tiles of a k_linear_wide workgroup, or 0 for
 // k_linear_mfma.
 //
@@ -872,28 +927,38 @@ bool lm_vec(const LinMfmaArgs& a) {  // k_linear_mfma's 16-byte loads
 // -> 256 31.6 -> 34.0): an eighth there (32768 x 1024 -> 1024 175 -> 146).
 // Past one round, the rounds at least three quarters full (100352 x 384 ->
 // 384, 0.94: 122 -> 87; 75000 x 384 -> 384, 0.71: 64.3 with k_linear_mfma).
-template <typename TIn>
-int lw_row_tiles(const LinMfmaArgs& a) {
-  if ((int64_t)a.c_out * a.kp * 2 >= (1ll << 31)) return 0;  // the buffer offsets' range
-  const int64_t cb = (a.c_out + kLwCols - 1) / kLwCols, cus = num_cus();
+//
+// And only where the estimates agree, since columns dropped, rows of y off a
+// 64-byte line and a short k add up differently from shape to shape: f16
+// 56000 x 132 -> 128 19.1 / 26.4, 65536 x 164 -> 128 23.8 / 29.4; f32 60000 x 164
+// -> 400 43.0 / 58.9, 65536 x 132 -> 128 22.4 / 30.3, 16384 x 256 -> 1420 52.0 /
+// 73.7 (k_linear_mfma / wide).
+int lw_row_tiles(const LinShape& s) {
+  if ((int64_t)s.c_out * lin_blocks(s.k, kLmK) * kLmK * 2 >= (1ll << 31)) return 0;  // the buffer offsets' range
+  const int64_t cb = lin_blocks(s.c_out, kLwCols), cus = s.cus;
   int rt = 0;
   int64_t best = 0, tiles = 0;
   for (const int r : {4, 8, 13}) {
-    const int64_t t = (a.m + 16 * r - 1) / (16 * r) * cb, cost = (t + cus - 1) / cus * (4 + r);
+    const int64_t t = lin_blocks(s.m, 16 * r) * cb, cost = lin_blocks(t, cus) * (4 + r);
     if (rt == 0 || cost < best) {
       rt = r;
       best = cost;
       tiles = t;
     }
   }
-  if (!lm_vec<TIn>(a)) {
-    if (tiles <= cus) return (a.c_out >= 128 && a.k >= 48) || rt == 4 || a.k >= 192 ? rt : 0;
-    return a.c_out >= 128 && a.k >= 48 && (a.k % 4 == 0 || a.k >= 160) ? rt : 0;
+  bool wide;
+  if (!s.vec) {
+    wide = tiles <= cus ? (s.c_out >= 128 && s.k >= 48) || rt == 4 || s.k >= 192
+                        : s.c_out >= 128 && s.k >= 48 && (s.k % 4 == 0 || s.k >= 160);
+  } else if (s.k < 192) {
+    wide = false;
+  } else if (rt == 4 && tiles <= cus) {
+    wide = 2 * cb * kLwCols <= 3 * (int64_t)s.c_out;
+  } else {
+    wide = 8 * cb * kLwCols <= 9 * (int64_t)s.c_out &&
+           (tiles <= cus || 4 * tiles >= 3 * cus * ((tiles + cus - 1) / cus));
   }
-  if (a.k < 192) return 0;
-  if (rt == 4 && tiles <= cus) return 2 * cb * kLwCols <= 3 * (int64_t)a.c_out ? rt : 0;
-  if (8 * cb * kLwCols > 9 * (int64_t)a.c_out) return 0;
-  return tiles <= cus || 4 * tiles >= 3 * cus * ((tiles + cus - 1) / cus) ? rt : 0;
+  return wide && lw_us(s, rt) < lm_us(s) ? rt : 0;
 }
 
 template <typename TIn, typename TOut, int RT, bool VEC>
@@ -936,7 +1001,7 @@ int launch_lb_d(const LinMfmaArgs& a, const uint32_t* bits, const uint32_t* flag
 
 template <typename TIn>
 int launch_lm_d(const LinMfmaArgs& a, int out_dtype, hipStream_t stream) {
-  const int rt = lw_row_tiles<TIn>(a);
+  const int rt = lw_row_tiles(lin_shape(a.m, a.k, a.c_out, sizeof(TIn) == 4 ? SF_F32 : SF_F16, a.x));
   if (rt != 0) return out_dtype == SF_F32 ? launch_lw<TIn, float>(a, rt, stream) : launch_lw<TIn, TIn>(a, rt, stream);
   const int64_t rbs = (a.m + kLmRows - 1) / kLmRows;
   const int64_t grid = rbs * ((a.c_out + kLmCols - 1) / kLmCols);
@@ -958,6 +1023,37 @@ int launch_lm_d(const LinMfmaArgs& a, int out_dtype, hipStream_t stream) {
 }  // namespace
 
 int linear_mfma_max_kp() { return kLmMaxK; }
+
+int linear_mfma_row_tiles(const void* x, int in_dtype, int64_t m, int k, int c_out) {
+  return lw_row_tiles(lin_shape(m, k, c_out, in_dtype, x));
+}
+
+// Whether the row prescan and k_linear_bits_mfma beat the direct kernels: from
+// outputs twice as wide as the input on, the large ones as measured here and
+// the others by the estimates (us, bitmap / direct, 10% spikes):
+//   f32   50176 x 384 -> 1536  153 / 165    32768 x 512 -> 2048  146 / 184
+//         65536 x 192 -> 768   63 / 71      65536 x 160 -> 1280  92 / 132
+//         25088 x 384 -> 1536  81 / 71      8192 x 512 -> 2048   50 / 46
+//         4096 x 1024 -> 4096  81 / 73      1000 x 384 -> 1536   29 / 15
+//         65536 x 128 -> 512   42 / 36      65536 x 128 -> 1536  93 / 143
+//         8192 x 768 -> 3072   98 / 85      10000 x 64 -> 256    16 / 7
+//   f16   50176 x 384 -> 1536  158 / 157    8192 x 512 -> 2048   80 / 50
+//         65536 x 192 -> 768   72 / 79      8192 x 768 -> 3072   153 / 89
+//         65536 x 128 -> 512   42 / 52      32768 x 128 -> 512   31 / 28
+//   f32, k no multiple of 16 or x off 16 bytes
+//         50176 x 385 -> 1536  172 / 216    58638 x 192 -> 744   71 / 122
+//         30000 x 132 -> 772   37 / 49      16384 x 50 -> 820    21 / 24
+//         66745 x 68 -> 324    36 / 47      8192 x 128 -> 1716   25 / 39
+// (x of full precision is faster direct throughout: 50176 x 384 -> 1536 408 /
+// 239.)  On binary x both give the same bits.
+bool linear_mfma_bits_pays(const void* x, int in_dtype, int64_t m, int k, int c_out) {
+  if (c_out < 2 * k || m * (int64_t)linear_words_per_row(k) * 4 >= (1ll << 31)) return false;
+  const LinShape s = lin_shape(m, k, c_out, in_dtype, x);
+  if (k < 192 ? !s.vec && m * c_out >= 25000000 : m * c_out >= 45000000) return true;
+  // Two launches instead of one: the host needs about 30 us for them.
+  const int rt = lw_row_tiles(s);
+  return 1.03 * (rt != 0 ? lw_us(s, rt) : lm_us(s)) >= std::max(lb_us(s), 30.0);
+}
 
 int launch_linear_bits_mfma(const LinMfmaArgs& a, const uint32_t* bits, const uint32_t* flags, int cwp, int in_dtype,
                             int out_dtype, hipStream_t stream) {

@@ -10,6 +10,7 @@ from pathlib import Path
 
 import numpy as np
 import pytest
+import torch
 
 from sparseflow_amd import _lib
 
@@ -320,3 +321,50 @@ def test_launch_plan_known_shapes():
     d = _lib.conv_desc(4, 64, 8, 8, 64, 8, 8, 1, 1, 0, 0, 0)
     with pytest.raises(_lib.UnsupportedError):
         _lib.conv2d_launch_plan(d)
+
+
+# ---- which Linear kernel a shape takes -----------------------------------------
+
+F32, F16, BF16 = torch.float32, torch.float16, torch.bfloat16
+
+# (m, k, c_out, dtype, offset of x past 16 bytes, the fastest of "tiles" (128 x
+# 128), "wide" (384 columns) and "bitmap", by a quarter or more unless noted,
+# binary x).
+LINEAR_ROUTES = [
+    # wide: the aligned shapes that fill its tiles, 16-bit and ragged x
+    (50176, 1536, 384, F32, 0, "wide"), (50176, 384, 384, F32, 0, "wide"), (3136, 768, 1152, F32, 0, "wide"),
+    (50176, 384, 384, F16, 0, "wide"), (8192, 512, 768, BF16, 0, "wide"), (50176, 1535, 384, F32, 0, "wide"),
+    (1000, 383, 384, F32, 0, "wide"), (8192, 512, 768, F32, 4, "wide"), (701, 1790, 100, F16, 0, "wide"),
+    (200, 1001, 12, F32, 0, "wide"), (34277, 742, 1456, F16, 0, "wide"),
+    # tiles: columns past the next 384 that are not there, short k
+    (65536, 132, 128, F32, 0, "tiles"), (56000, 132, 128, F16, 0, "tiles"), (65536, 164, 128, F16, 0, "tiles"),
+    (65536, 512, 512, F32, 0, "tiles"), (100000, 128, 128, F32, 0, "tiles"), (65536, 129, 128, F32, 0, "tiles"),
+    (40000, 384, 256, F32, 0, "tiles"), (112945, 64, 96, F16, 0, "tiles"),
+    # bitmap: outputs from twice the input on, large or with columns to spare
+    (50176, 384, 1536, F32, 0, "bitmap"), (32768, 512, 2048, F32, 0, "bitmap"), (65536, 160, 1280, F32, 0, "bitmap"),
+    (65536, 128, 1536, F32, 0, "bitmap"), (58638, 192, 744, F32, 4, "bitmap"), (30000, 132, 772, F32, 0, "bitmap"),
+    (66745, 68, 324, F32, 0, "bitmap"), (60774, 111, 320, F32, 0, "bitmap"), (31712, 157, 604, F32, 0, "bitmap"),
+    (25088, 395, 1732, F32, 0, "bitmap"), (56000, 200, 772, F32, 0, "bitmap"),
+    # direct although the output is wide: small calls
+    (1000, 384, 1536, F32, 0, "wide"), (8192, 768, 2048, F16, 0, "wide"), (10000, 64, 256, F32, 0, "tiles"),
+]
+
+
+@pytest.mark.parametrize("case", LINEAR_ROUTES)
+def test_linear_route(case):
+    m, k, c_out, dtype, offset, want = case
+    bits = _lib.linear_mfma_bits_pays(m, k, c_out, dtype, offset)
+    tiles = _lib.linear_mfma_row_tiles(m, k, c_out, dtype, offset)
+    assert tiles in (0, 4, 8, 13)
+    assert ("bitmap" if bits else "wide" if tiles else "tiles") == want
+
+
+# Every shape gets a kernel that takes it: W's rows within the 31-bit buffer
+# offsets of the wide kernel, x's bitmap below 2^31 bytes.
+def test_linear_route_limits():
+    assert _lib.linear_mfma_row_tiles(300, 8192, 131072, F16) == 0
+    assert _lib.linear_mfma_row_tiles(300, 8192, 131068, F16) > 0
+    assert not _lib.linear_mfma_bits_pays(1 << 28, 40, 128, F16)
+    assert _lib.linear_mfma_bits_pays((1 << 28) - 1, 40, 128, F16)
+    for m, k, c in ((0, 64, 64), (64, 0, 64), (64, 64, 0)):
+        assert _lib.linear_mfma_row_tiles(m, k, c, F32) == 0 and not _lib.linear_mfma_bits_pays(m, k, c, F32)

@@ -244,11 +244,15 @@ def test_linear_random_shapes(case, kernel):
 # The 384-column kernel: tiles of 64, 128 and 208 rows (by how many fill 256
 # CUs), rows and columns on both sides of a tile's end, k with and without a
 # remainder of 32 and of 4, an odd number of K steps, x of one bit and of full
-# precision, x that starts one element past 16 bytes.  f32 x with k = 176 takes
-# it only from such a start, 53249 rows of k = 50 never do.
-WIDE_CASES = [(1, 192, 384), (64, 196, 260), (65, 384, 388), (16384, 224, 384), (16385, 224, 768), (32768, 192, 384),
-              (32769, 256, 384), (53249, 193, 384), (208 * 256, 192, 1536), (70, 194, 384), (70, 176, 384),
-              (300, 48, 128), (300, 3, 4), (300, 44, 124), (209, 51, 132), (53249, 50, 128), (9, 415, 1000)]
+# precision, x that starts one element past 16 bytes.  Expected: the row tiles
+# of aligned f32, f32 from such a start, and 16-bit x (0: the 128 x 128 kernel).
+WIDE_TILES = {(1, 192, 384): (4, 4, 4), (64, 196, 260): (4, 4, 4), (65, 384, 388): (0, 4, 4),
+              (16384, 224, 384): (4, 4, 4), (16385, 224, 768): (13, 13, 13), (25087, 384, 384): (8, 8, 8),
+              (32768, 192, 384): (0, 8, 8), (32769, 256, 384): (13, 13, 13), (53249, 193, 384): (8, 8, 8),
+              (208 * 256, 192, 1536): (0, 13, 13), (70, 194, 384): (4, 4, 4), (70, 176, 384): (0, 4, 4),
+              (300, 48, 128): (0, 4, 4), (300, 3, 4): (0, 0, 0), (300, 44, 124): (4, 4, 4), (209, 51, 132): (4, 4, 4),
+              (53249, 50, 128): (0, 0, 0), (9, 415, 1000): (4, 4, 4)}
+WIDE_CASES = list(WIDE_TILES)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
@@ -266,6 +270,10 @@ def test_mfma_wide_tiles(case, form, dtype):
         x[m // 2, k - 1] = float("inf")
     w = _w(co, k, seed=co).to(DEV)
     b = (torch.randn(co, generator=torch.Generator().manual_seed(34)) * 0.1).to(DEV)
+    aligned, offset, half_x = WIDE_TILES[case]
+    size = x.element_size()
+    assert _lib.linear_mfma_row_tiles(m, k, co, dtype, 0) == (aligned if size == 4 else half_x)
+    assert _lib.linear_mfma_row_tiles(m, k, co, dtype, size) == (offset if size == 4 else half_x)
     y, kernels = _run(x, w, b, kernel="mfma", threshold=1e-6, output_dtype=torch.float32)
     assert set(kernels) == {"linear_mfma"}, kernels
     off = torch.empty(m * k + 1, device=DEV, dtype=dtype)[1:].view(m, k).copy_(x)
