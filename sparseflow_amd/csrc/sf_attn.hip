@@ -79,7 +79,7 @@ __global__ __launch_bounds__(64 * kAttnWaves) void k_spike_attn(AttnArgs a) {
   const int n = lane % MT, kk = lane / MT;
   const int S = a.s;
   const int64_t items = a.tb * (int64_t)a.h;
-  const int64_t item = W == 1 ? (int64_t)blockIdx.x * kAttnWaves + wave : (int64_t)blockIdx.x;
+  const int64_t item = a.item0 + (W == 1 ? (int64_t)blockIdx.x * kAttnWaves + wave : (int64_t)blockIdx.x);
   const int part = W == 1 ? 0 : wave;
   if (item >= items) return;  // W == 1 only: a whole wavefront, and no barrier follows there
   const int64_t tbi = item / a.h;
@@ -234,19 +234,21 @@ __global__ __launch_bounds__(64 * kAttnWaves) void k_spike_attn(AttnArgs a) {
 }
 
 template <typename T, typename TOut, int D, int W>
-int launch_attn_w(const AttnArgs& a, hipStream_t stream) {
-  const int64_t items = a.tb * (int64_t)a.h;
-  const int64_t grid = W == 1 ? (items + kAttnWaves - 1) / kAttnWaves : items;
-  if (grid == 0) return (int)hipSuccess;
-  if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
+int launch_attn_w(AttnArgs a, hipStream_t stream) {
   // q's four-element loads: its base and row starts at multiples of them.
   const bool vec = ((reinterpret_cast<uintptr_t>(a.q) / sizeof(T)) | (uintptr_t)(a.s_tb | a.s_m | a.s_h)) % 4 == 0;
-  if (vec)
-    hipLaunchKernelGGL((k_spike_attn<T, TOut, D, W, true>), dim3((unsigned)grid), dim3(64 * kAttnWaves), 0, stream, a);
-  else
-    hipLaunchKernelGGL((k_spike_attn<T, TOut, D, W, false>), dim3((unsigned)grid), dim3(64 * kAttnWaves), 0, stream,
-                       a);
-  return (int)hipGetLastError();
+  // (A launch holds fewer than 2^32 threads.)
+  constexpr int64_t kLaunchItems = (int64_t)1 << 24;
+  const int64_t items = a.tb * (int64_t)a.h;
+  for (a.item0 = 0; a.item0 < items; a.item0 += kLaunchItems) {
+    const int64_t n = items - a.item0 < kLaunchItems ? items - a.item0 : kLaunchItems;
+    const dim3 grid((unsigned)(W == 1 ? (n + kAttnWaves - 1) / kAttnWaves : n)), block(64 * kAttnWaves);
+    if (vec) hipLaunchKernelGGL((k_spike_attn<T, TOut, D, W, true>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((k_spike_attn<T, TOut, D, W, false>), grid, block, 0, stream, a);
+    const int rc = (int)hipGetLastError();
+    if (rc != (int)hipSuccess) return rc;
+  }
+  return (int)hipSuccess;
 }
 
 template <typename T, typename TOut, int D>

@@ -260,6 +260,7 @@ struct AttnArgs {
   int s, h, d;
   int64_t s_tb, s_m, s_h;  // q / k / v strides (elements)
   int64_t y_tb, y_m, y_h;  // y strides
+  int64_t item0;           // first (frame, head) item of the launch
   float scale, cutoff;
 };
 size_t attn_lds_bytes(int s, int d);

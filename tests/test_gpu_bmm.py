@@ -225,6 +225,20 @@ def test_fused_spike_attention_non_finite_rows(shape, bad):
     assert ok, f"max abs err {err}"
 
 
+# More (frame, head) items than one launch has threads for (2^32, a wavefront
+# each).  Sums of at most 16 ones, times 1/4: exact.
+def test_fused_spike_attention_very_many_items():
+    from sparseflow_amd.Kernels.attention import sparse_spike_attention_forward
+
+    shape = (2 ** 22 + 3, 16, 1, 16)
+    announce(f"spike attention many items {shape}")
+    g = torch.Generator(device=DEV).manual_seed(29)
+    q, k, v = (torch.empty(shape, device=DEV, dtype=torch.float16).bernoulli_(0.3, generator=g) for _ in range(3))
+    y = sparse_spike_attention_forward(q, k, v)
+    ref = (q * k).sum(-1, keepdim=True) * v * 0.25
+    assert torch.equal(y, ref)
+
+
 def test_fused_spike_attention_unsupported_shapes():
     from sparseflow_amd.Kernels.attention import sparse_spike_attention_forward
 
