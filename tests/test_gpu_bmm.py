@@ -178,6 +178,14 @@ def test_fused_spike_attention(shape, p):
     assert torch.equal(yt.transpose(1, 2).cpu(), y.cpu())
 
 
+def _rounded_tol(dtype):
+    """FP32_TOL and one rounding of the result to dtype (11 or 8 bits; f16
+    below 2^-14: 2^-25)."""
+    half = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    return {"atol": FP32_TOL["atol"] * (1 + half) + (2.0 ** -25 if dtype == torch.float16 else 0.0),
+            "rtol": FP32_TOL["rtol"] * (1 + half) + half}
+
+
 # Edges of the matrix-core form: rows below and around a K step, a batch of
 # loads and a row tile, for each head_dim; real values (f32 sums of at most
 # 300 + 64 products: relative error below 400 * 2^-24); q rows that are not
@@ -185,18 +193,21 @@ def test_fused_spike_attention(shape, p):
 @pytest.mark.parametrize("shape", [(2, 3, 1, 32), (2, 3, 3, 16), (1, 2, 17, 64), (2, 2, 33, 32), (1, 3, 65, 16),
                                    (2, 2, 287, 64), (260, 8, 9, 32), (520, 4, 5, 64), (260, 8, 6, 16)])
 @pytest.mark.parametrize("aligned", [True, False])
-def test_fused_spike_attention_edges(shape, aligned):
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_fused_spike_attention_edges(shape, aligned, dtype):
     from sparseflow_amd.Kernels.attention import sparse_spike_attention_forward
 
     B, H, S, D = shape
     g = torch.Generator().manual_seed(25)
     pad = 0 if aligned else 1
-    q, k, v = (torch.randn(B, H, S, D + pad, generator=g)[..., pad:] for _ in range(3))
-    announce(f"spike attention edges {shape} aligned={aligned}")
-    ref = torch.matmul(torch.matmul(olin.masked(q, 0.5).double(), k.double().transpose(-2, -1)) * D ** -0.5, v.double())
-    dq, dk, dv = (torch.randn(B, H, S, D + pad, device=DEV)[..., pad:].copy_(t) for t in (q, k, v))
+    q, k, v = (torch.randn(B, H, S, D + pad, generator=g)[..., pad:].to(dtype) for _ in range(3))
+    announce(f"spike attention edges {shape} aligned={aligned} {dtype}")
+    ref = torch.matmul(torch.matmul(olin.masked(q.float(), 0.5).double(), k.double().transpose(-2, -1)) * D ** -0.5,
+                       v.double())
+    dq, dk, dv = (torch.randn(B, H, S, D + pad, device=DEV).to(dtype)[..., pad:].copy_(t) for t in (q, k, v))
     y = sparse_spike_attention_forward(dq, dk, dv, threshold=0.5)
-    ok, err, _ = close(y, ref, **FP32_TOL)
+    assert y.dtype == dtype
+    ok, err, _ = close(y, ref, **_rounded_tol(dtype))
     assert ok, f"max abs err {err}"
 
 
@@ -204,24 +215,25 @@ def test_fused_spike_attention_edges(shape, aligned):
 # is active.
 @pytest.mark.parametrize("shape", [(1, 2, 40, 16), (1, 2, 40, 32), (1, 2, 40, 64), (260, 8, 40, 32)])
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
-def test_fused_spike_attention_non_finite_rows(shape, bad):
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_fused_spike_attention_non_finite_rows(shape, bad, dtype):
     from sparseflow_amd.Kernels.attention import sparse_spike_attention_forward
 
-    q, k, v = (spikes(shape, 0.3, seed=s) for s in (26, 27, 28))
+    q, k, v = (spikes(shape, 0.3, seed=s, dtype=dtype) for s in (26, 27, 28))
     D = shape[3]
     d = D - 3
     k[0, 1, 5, :] = 0.0
     k[0, 1, 5, d] = 1.0
     v[0, 1, 5, 2] = bad        # KV[d][2]; the other KV[.][2] meet 0 * bad
-    announce(f"spike attention non-finite {shape} {bad}")
+    announce(f"spike attention non-finite {shape} {bad} {dtype}")
     y = sparse_spike_attention_forward(q.to(DEV), k.to(DEV), v.to(DEV)).cpu()
     fine = torch.isfinite(y)
     expect = torch.ones(shape, dtype=torch.bool)
-    expect[0, 1, :, 2] = q[0, 1].sum(-1) == 0     # every KV[.][2] is inf or NaN
+    expect[0, 1, :, 2] = q[0, 1].float().sum(-1) == 0     # every KV[.][2] is inf or NaN
     assert torch.equal(fine, expect)
     ref = torch.matmul(torch.matmul(q.double(), k.double().transpose(-2, -1)) * D ** -0.5,
                        torch.nan_to_num(v, nan=0.0, posinf=0.0).double())
-    ok, err, _ = close(y[fine], ref[fine], **FP32_TOL)
+    ok, err, _ = close(y[fine], ref[fine], **_rounded_tol(dtype))
     assert ok, f"max abs err {err}"
 
 
