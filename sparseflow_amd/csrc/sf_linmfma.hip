@@ -578,7 +578,7 @@ __global__ __launch_bounds__(64 * kLbWaves, 2) void k_linear_bits_mfma(LinMfmaAr
           c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[rt], bh[ct], c, 0, 0, 0);
         }
       }
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // the tiles of step s + 1 (the x loads are waited for already)
+      lds_dma_wait();  // the tiles of step s + 1: the compiler does not count them
       __syncthreads();
     }
   }
