@@ -594,8 +594,11 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const
     const int g = t * 64 + lane;
     const bool mine = tile < nt && g < total_px;
     const int gc = mine ? g : total_px - 1;  // lanes past the end form valid addresses
-    const int sample = gc / hwo;
-    const int q = gc - sample * hwo;
+    // (opaque: the division's reciprocal, formed ahead of the loop, was spilled)
+    int hwo_d = hwo;
+    asm volatile("" : "+s"(hwo_d));
+    const int sample = gc / hwo_d;
+    const int q = gc - sample * hwo_d;
     const int oh = q / a.w_out, ow = q - (q / a.w_out) * a.w_out;
     const int ih0 = oh * a.s - 1, iw0 = ow * a.s - 1;
     const uint32_t fbase = (uint32_t)sample * frame_bytes;
