@@ -422,7 +422,7 @@ int sf_bmm_sparse(const void* a, const void* b, int32_t in_dtype, int64_t batche
  * tb*qkv_strides[0] + m*qkv_strides[1] + h*qkv_strides[2] + d, of y at the
  * same form with y_strides (elements; d contiguous).  q elements with
  * f16(|q|) <= f16(threshold) count as zero.  head_dim d in {16, 32, 64};
- * supported while sf_spike_attention_supported(s, d).  No counterpart entry
+ * s up to 1271, 623 and 287 (sf_spike_attention_supported).  No counterpart entry
  * point in the reference (it runs the two stages as separate bmm calls). */
 int sf_spike_attention_supported(int32_t s, int32_t d);
 int sf_spike_attention(const void* q, const void* k, const void* v,

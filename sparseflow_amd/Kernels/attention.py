@@ -56,8 +56,9 @@ def sparse_spike_attention_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Te
     token_major=False: q, k, v [B, heads, seq, head_dim] -> y of that shape.
     token_major=True:  q, k, v [B, seq, heads, head_dim] (the projections'
     [B, seq, dim] output viewed per head) -> y [B, seq, heads, head_dim].
-    Returns None when the kernel does not take the shape (head_dim not in
-    {16, 32, 64} or k, v do not fit in LDS): the caller runs the two stages."""
+    Returns None when sf_spike_attention does not take the shape (head_dim not
+    in {16, 32, 64}, or more than 1271, 623 or 287 tokens): the caller runs the
+    two stages."""
     from .. import _lib
 
     if not q.is_cuda or q.dtype not in (torch.float32, torch.float16, torch.bfloat16):

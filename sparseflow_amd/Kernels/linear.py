@@ -210,6 +210,7 @@ def sparse_linear_forward(
         if w_split is None or tuple(w_split[0].shape) != (C_OUT, -(-C_IN // 32) * 32):
             w_split = split_weight_bf16(weight)
         meta["reason"] = "linear_mfma_bitmap" if mfma_bits else "linear_mfma_bf16x2"
+        # 128 x 128 pieces of the output, whichever kernel's tiles cover them.
         meta["launch_count"] = int(-(-N // 128) * -(-C_OUT // 128))
     if use_mfma and not need_stats:
         if return_ms:

@@ -12,19 +12,22 @@
 // k and of v per half wavefront (two 128-byte runs per load at D = 32), and
 // KV, as the first product leaves it in the accumulators (lane = column e,
 // register = row d), is the second product's B operand as it stands, with
-// q's four-element pieces as the A operand.  Nothing is staged in LDS, no
-// wavefront waits for another, and the loads of the next K steps and of the
-// next rows of q are in flight during the MFMAs.  q elements below the
+// q's four-element pieces as the A operand.  q, k and v are not staged in LDS,
+// and the loads of the next K steps and of the next rows of q are in flight
+// during the MFMAs.  With enough items a wavefront takes one and waits for no
+// other; with few, four wavefronts share an item's rows and add their partial
+// sums of KV through LDS, behind the one barrier.  q elements below the
 // activity cutoff count as zero (the reference's prescan test on the left
 // operand).  Sums run in an order fixed by the shape: deterministic.
 //
 // Bound by HBM (q, k, v in, y out).  At 256 frames x 12 heads x 196 tokens x
-// 32 (308 MB): 63.3 us = 4.9 TB/s, the
-// card's copy rate; the form before it, which staged k and v in LDS as f32
-// and formed KV and the rows on the VALU, took 133.5 us.
+// 32 (308 MB), inputs new at every call: 64 us = 4.8 TB/s, the card's copy rate
+// (the same inputs again, partly in the last-level cache: 52 us); the form before it, which staged k
+// and v in LDS as f32 and formed KV and the rows on the VALU, took 127 us.
 //
-// An item whose KV is not finite everywhere takes walk_rows instead: there
-// an inactive q element must not meet a KV row (0 * inf would be NaN).
+// An item whose KV is not finite everywhere takes its q rows' active elements
+// one by one instead: there an inactive one must not meet a KV row (0 * inf
+// would be NaN).
 //
 // Layout: element (tb, m, h, d) at tb*s_tb + m*s_m + h*s_h + d for q, k, v
 // (one set of strides) and for y (its own), so both token-major
@@ -278,7 +281,9 @@ int launch_attn_d(const AttnArgs& a, int out_dtype, hipStream_t stream) {
 
 }  // namespace
 
-size_t attn_lds_bytes(int s, int d) { return ((size_t)2 * s * d + (size_t)d * (d + 1)) * sizeof(float); }
+// Head widths of the matrix cores' tiles.  The lengths are the declared range of
+// the entry point; the kernel itself has no limit on them.
+int attn_max_tokens(int d) { return d == 16 ? 1271 : d == 32 ? 623 : d == 64 ? 287 : 0; }
 
 int launch_spike_attn(const AttnArgs& a, int in_dtype, int out_dtype, hipStream_t stream) {
   timing_begin(K_ATTN, stream);

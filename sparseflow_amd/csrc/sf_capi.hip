@@ -687,7 +687,7 @@ int sf_bmm_sparse(const void* a, const void* b, int32_t in_dtype, int64_t batche
 // ---- fused spike attention ----------------------------------------------------
 
 int sf_spike_attention_supported(int32_t s, int32_t d) {
-  return s >= 1 && (d == 16 || d == 32 || d == 64) && sf::attn_lds_bytes(s, d) <= (size_t)sf::kMaxLdsBytes;
+  return s >= 1 && s <= sf::attn_max_tokens(d);
 }
 
 int sf_spike_attention(const void* q, const void* k, const void* v, int32_t in_dtype, int64_t tb, int32_t s,
@@ -698,7 +698,7 @@ int sf_spike_attention(const void* q, const void* k, const void* v, int32_t in_d
   if (out_dtype != in_dtype && out_dtype != SF_F32)
     return fail(SF_ERR_UNSUPPORTED, "out_dtype must equal in_dtype or be f32");
   if (!sf_spike_attention_supported(s, d))
-    return fail(SF_ERR_UNSUPPORTED, "head_dim must be 16, 32 or 64 and 2*s*d + d*(d+1) floats fit 160 KB of LDS");
+    return fail(SF_ERR_UNSUPPORTED, "head_dim must be 16, 32 or 64, with at most 1271, 623 or 287 tokens");
   if (qkv_strides == nullptr || y_strides == nullptr) return fail(SF_ERR_INVALID, "NULL strides");
   if (tb == 0) return SF_OK;
   if (q == nullptr || k == nullptr || v == nullptr || y == nullptr) return fail(SF_ERR_INVALID, "NULL pointer");

@@ -263,7 +263,7 @@ struct AttnArgs {
   int64_t item0;           // first (frame, head) item of the launch
   float scale, cutoff;
 };
-size_t attn_lds_bytes(int s, int d);
+int attn_max_tokens(int d);  // of a supported head_dim d, otherwise 0
 int launch_spike_attn(const AttnArgs& a, int in_dtype, int out_dtype, hipStream_t stream);
 
 // Raise kernel K's dynamic-LDS ceiling to `bytes` (the default limit is

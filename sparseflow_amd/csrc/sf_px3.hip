@@ -535,11 +535,11 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3(ConvArgs a, const 
 // (chunk, tap, ci) order, as there.
 // ---------------------------------------------------------------------------
 
-// Direct-to-LDS loads of chunk c by the nw wavefronts of the workgroup.
-__device__ __forceinline__ void load_chunk_px3_nw(char* buf, const float* __restrict__ wt, int c, int krows,
-                                                  int c_out, int co0, int wave, int nw, int lane) {
+// load_chunk_px3<64> as a loop: a unit's addresses at a time.
+__device__ __forceinline__ void load_chunk_px3s(char* buf, const float* __restrict__ wt, int c, int krows, int c_out,
+                                                int co0, int wave, int lane) {
   typedef Px3Layout<64> L;
-  for (int u = wave; u < L::units; u += nw) {
+  for (int u = wave; u < L::units; u += kRowsWaves) {
     const int pos = u * 64 + lane;
     const int r = pos / L::stride;
     const int q = pos - r * L::stride;
@@ -566,7 +566,6 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const
   extern __shared__ __align__(16) char smem[];
   __shared__ float s_seed[64];
   __shared__ uint32_t s_queued[kRowsWaves];  // per tile: on the dense queue
-  constexpr int nw = kRowsWaves;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tile = SPLIT == 1 ? wave : wave / SPLIT;  // of the workgroup's nt; past them: a wavefront that only loads
   const int part = SPLIT == 1 ? 0 : wave % SPLIT;     // its channels: CW part ..
@@ -648,7 +647,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const
     {
       int ll = lane;
       asm volatile("" : "+v"(ll));
-      load_chunk_px3_nw(smem, wt, 0, krows, a.c_out, co0, wave, nw, ll);
+      load_chunk_px3s(smem, wt, 0, krows, a.c_out, co0, wave, ll);
     }
     if (SPLIT > 1 && dense && s_queued[tile] != 0u) {
       walk = false;
@@ -665,7 +664,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_conv_px3s(ConvArgs a, const
       if (c + 1 < nchunks) {
         int ll = lane;
         asm volatile("" : "+v"(ll));
-        load_chunk_px3_nw(smem + ((c + 1) & 1) * LY::chunk_bytes, wt, c + 1, krows, a.c_out, co0, wave, nw, ll);
+        load_chunk_px3s(smem + ((c + 1) & 1) * LY::chunk_bytes, wt, c + 1, krows, a.c_out, co0, wave, ll);
       }
       uint32_t w[9];
 #pragma unroll

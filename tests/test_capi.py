@@ -156,9 +156,12 @@ def test_linear_bmm_attention_sizes_and_validation():
     assert L.sf_bmm_sparse(p, p, 0, 2, 4, 300, 8, 0, 1, 300, 1e-6, 1.0, p, 0, None) == _lib.SF_ERR_UNSUPPORTED
     assert L.sf_bmm_sparse(p, p, 0, 0, 4, 30, 8, 0, 8, 1, 1e-6, 1.0, p, 0, None) == _lib.SF_OK
     assert L.sf_bmm_sparse(p, p, 0, 2, 4, 30, 8, 0, -1, 1, 1e-6, 1.0, p, 0, None) == _lib.SF_ERR_INVALID
-    # Fused attention: head_dim 16/32/64 and k, v within LDS.
+    # Fused attention: head_dim 16/32/64 and the declared lengths.
     assert L.sf_spike_attention_supported(196, 32) and not L.sf_spike_attention_supported(196, 48)
     assert not L.sf_spike_attention_supported(700, 64)
+    for d, s in ((16, 1271), (32, 623), (64, 287)):
+        assert L.sf_spike_attention_supported(s, d) and L.sf_spike_attention_supported(1, d)
+        assert not L.sf_spike_attention_supported(s + 1, d) and not L.sf_spike_attention_supported(0, d)
     st = (ctypes.c_int64 * 3)(0, 0, 0)
     assert L.sf_spike_attention(p, p, p, 0, 2, 196, 12, 48, st, 0.2, 1e-6, p, st, 0, None) == _lib.SF_ERR_UNSUPPORTED
     assert L.sf_spike_attention(p, p, p, 0, 0, 196, 12, 32, st, 0.2, 1e-6, p, st, 0, None) == _lib.SF_OK

@@ -257,5 +257,5 @@ def test_fused_spike_attention_unsupported_shapes():
     q = spikes((2, 2, 20, 48), 0.1, seed=23).to(DEV)
     assert sparse_spike_attention_forward(q, q, q) is None          # head_dim 48
     q = spikes((1, 1, 700, 64), 0.1, seed=24).to(DEV)
-    assert sparse_spike_attention_forward(q, q, q) is None          # k, v exceed LDS
+    assert sparse_spike_attention_forward(q, q, q) is None          # past the declared lengths
     assert not _lib.spike_attention_supported(700, 64) and _lib.spike_attention_supported(196, 32)
