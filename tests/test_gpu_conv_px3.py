@@ -296,16 +296,24 @@ def test_px3_random_shapes(case):
 # walked by four wavefronts, a quarter of the channels each) and five and more
 # (one wavefront); channel groups that end inside a wavefront's quarter; dense
 # tiles beside walked ones.  C_in > 128 (streamed), up to 128 and up to 64.
-SPLIT_CASES = [(1, 132, 1, 1, 20, 1), (2, 160, 5, 13, 4, 1), (64, 129, 16, 16, 64, 1), (65, 140, 16, 16, 76, 1),
-               (200, 136, 16, 16, 84, 1), (129, 150, 23, 22, 64, 2), (321, 130, 16, 16, 60, 1),
-               (1, 100, 1, 1, 20, 1), (2, 128, 5, 13, 36, 1), (64, 65, 16, 16, 64, 1), (200, 100, 15, 14, 76, 2),
-               (1, 20, 1, 1, 4, 1), (2, 40, 5, 13, 20, 1), (65, 64, 16, 16, 76, 1), (321, 33, 16, 16, 60, 1)]
+# Expected: tiles of a pass, wavefronts per tile.
+SPLIT_PLANS = {(1, 132, 1, 1, 20, 1): (1, 4), (2, 160, 5, 13, 4, 1): (1, 4), (64, 129, 16, 16, 64, 1): (1, 4),
+               (65, 140, 16, 16, 76, 1): (3, 4), (256, 129, 16, 16, 20, 1): (4, 4), (257, 129, 16, 16, 20, 1): (5, 1),
+               (200, 136, 16, 16, 84, 1): (7, 1), (129, 150, 23, 22, 64, 2): (2, 4), (321, 130, 16, 16, 60, 1): (6, 1),
+               (1, 100, 1, 1, 20, 1): (1, 4), (2, 128, 5, 13, 36, 1): (1, 4), (64, 65, 16, 16, 64, 1): (2, 4),
+               (200, 100, 15, 14, 76, 2): (3, 4), (100, 66, 16, 16, 76, 1): (5, 1),
+               (1, 20, 1, 1, 4, 1): (1, 4), (2, 40, 5, 13, 20, 1): (1, 4), (65, 64, 16, 16, 76, 1): (3, 4),
+               (256, 40, 16, 16, 20, 1): (4, 4), (321, 33, 16, 16, 60, 1): (6, 1)}
+SPLIT_CASES = list(SPLIT_PLANS)
 
 
 @pytest.mark.parametrize("case", SPLIT_CASES)
 @pytest.mark.parametrize("form", ["sparse", "dense tiles", "values"])
 def test_px3_tiles_split_over_wavefronts(case, form):
     N, C, H, W, Co, s = case
+    ho, wo = -(-H // s), -(-W // s)
+    plan = _lib.conv2d_launch_plan(_lib.conv_desc(N, C, H, W, Co, ho, wo, 3, s, 1, _lib.SF_F32, _lib.SF_F32))
+    assert plan[1:] == SPLIT_PLANS[case], plan
     announce(f"px3 split {case} {form}")
     g = torch.Generator(device=DEV).manual_seed(N + C)
     x = (torch.rand(N, C, H, W, generator=g, device=DEV) < 0.01).float()

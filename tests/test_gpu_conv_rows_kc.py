@@ -125,15 +125,18 @@ def test_rows_kc_deterministic_bitwise():
     assert torch.equal(y1, y2)
 
 
-# Tiles per workgroup as they spread over 256 CUs: 1 (a frame alone), 1, 4, 7
-# and 16, with the last workgroup's short.
-SPREAD_CASES = [(1, 130, 2, 28, 4), (3, 150, 14, 14, 64), (100, 130, 14, 14, 132), (64, 140, 28, 28, 68),
-                (290, 129, 28, 28, 60)]
+# Tiles per workgroup as they spread over 256 CUs: 1 (a frame alone), 1, 5, 7 and
+# 16, with the last workgroup's short; six channel groups; two rounds of the chip.
+SPREAD_TILES = {(1, 130, 2, 28, 4): 1, (3, 150, 14, 14, 64): 1, (100, 130, 14, 14, 132): 5, (64, 140, 28, 28, 68): 7,
+                (290, 129, 28, 28, 60): 16, (33, 130, 14, 14, 324): 4, (300, 129, 14, 14, 196): 10}
+SPREAD_CASES = list(SPREAD_TILES)
 
 
 @pytest.mark.parametrize("case", SPREAD_CASES)
 def test_rows_kc_tiles_spread_over_cus(case):
     N, C, H, W, Co = case
+    plan = _lib.conv2d_launch_plan(_lib.conv_desc(N, C, H, W, Co, H, W, 3, 1, 1, _lib.SF_F32, _lib.SF_F32))
+    assert plan[1:] == (SPREAD_TILES[case], 1), plan
     announce(f"rows_kc spread {case}")
     x = spikes((N, C, H, W), 0.01, seed=N + C)
     w, b = _weights(Co, C), torch.linspace(-0.3, 0.3, Co)

@@ -12,6 +12,7 @@ import torch
 import torch.nn as nn
 
 from oracle import conv as oconv, lif as olif
+from sparseflow_amd import _lib
 from sparseflow_amd.Kernels.fused_conv_lif import sparse_fused_conv_lif_forward, sparse_fused_conv_lif_multistep
 from sparseflow_amd.neuron import LIFNode
 from sparseflow_amd.Ops.sparse_fused_conv_lif import FusedSparseConvLIF
@@ -245,14 +246,19 @@ def test_fused_lif_pixel_kernel_random_shapes(case):
 
 # Tiles per workgroup as the pixel kernel spreads them over 256 CUs: one to
 # four (four wavefronts per tile where the weights stay resident, C_in <= 128)
-# and more; channel slices that end inside a wavefront's eight.
-SPREAD_CASES = [(3, 1, 20, 3, 5, 4), (2, 2, 128, 9, 13, 36), (2, 96, 64, 16, 16, 44), (2, 190, 33, 16, 14, 64),
-                (2, 2, 132, 9, 13, 36), (2, 96, 150, 16, 16, 44)]
+# and more; channel slices that end inside a wavefront's eight.  Expected: tiles
+# of a pass, wavefronts per tile.
+SPREAD_PLANS = {(3, 1, 20, 3, 5, 4): (1, 4), (2, 2, 128, 9, 13, 36): (1, 4), (2, 96, 64, 16, 16, 44): (3, 4),
+                (2, 190, 33, 16, 14, 64): (6, 1), (2, 2, 132, 9, 13, 36): (1, 1), (2, 96, 150, 16, 16, 44): (3, 1),
+                (2, 33, 140, 14, 14, 196): (4, 1)}
+SPREAD_CASES = list(SPREAD_PLANS)
 
 
 @pytest.mark.parametrize("case", SPREAD_CASES)
 def test_fused_lif_tiles_spread_over_cus(case):
     T, N, C, H, W, Co = case
+    plan = _lib.conv2d_launch_plan(_lib.conv_desc(N, C, H, W, Co, H, W, 3, 1, 1, _lib.SF_F32, _lib.SF_F32), True)
+    assert plan[1:] == SPREAD_PLANS[case], plan
     announce(f"lif spread {case}")
     x = spikes((T, N, C, H, W), 0.05, seed=N + C)
     w = torch.randn(Co, C, 3, 3, generator=torch.Generator().manual_seed(C)) * (4.0 / (C * 9)) ** 0.5 * 2.0
