@@ -62,6 +62,15 @@ constexpr int kPx3Rows = kPx3Ch * 9;     // weight rows per chunk
 // x 512 x 14 x 14 -> 512 stride 2 152.6 / 152.1, 158 x 319 x 44 x 44 -> 52 120 /
 // 115).
 constexpr int kPx3SplitTiles = 4;
+// Slices of 32 channels (64 < C_in <= 128, no LIF) leave a wavefront eight, too
+// few for the selection of their spike that each does for itself: three and
+// four tiles lose (us, one -> four walking wavefronts, 1% spikes: 60 / 95 / 125 x
+// 100 x 16 x 16 -> 64, two / three / four tiles, 15.1 -> 15.4, 15.1 -> 16.9, 15.3 ->
+// 19.4; at 3% 20.9 -> 20.2, 21.2 -> 23.7, 21.1 -> 28.0).  With the LIF's work
+// split too, the four gain there as well (4 x 63 x 128 x 14 x 14 -> 128, four
+// tiles, 72 -> 51).
+template <int CO, bool LIF>
+constexpr int px3w_split_tiles() { return CO == 32 && !LIF ? 2 : kPx3SplitTiles; }
 
 // LDS layout of a chunk for a workgroup slice of CO output channels.
 //  CO = 64: rows of 16 pieces (16 bytes = 4 channels) padded to 17 pieces
@@ -1066,8 +1075,8 @@ int launch_px3w_to(const ConvArgs& a, hipStream_t stream) {
   // of passes: no CU idles through another's last pass.
   const GroupSpread sp = px3w_spread<CO>(a);
   const int grid = groups * sp.per_group, nt = sp.waves;
-  return nt <= kPx3SplitTiles ? launch_px3w_cw<TIn, TOut, CO, LIF, CO / 4>(a, grid, groups, nt, stream)
-                              : launch_px3w_cw<TIn, TOut, CO, LIF, CO>(a, grid, groups, nt, stream);
+  return nt <= px3w_split_tiles<CO, LIF>() ? launch_px3w_cw<TIn, TOut, CO, LIF, CO / 4>(a, grid, groups, nt, stream)
+                                           : launch_px3w_cw<TIn, TOut, CO, LIF, CO>(a, grid, groups, nt, stream);
 }
 
 template <typename TIn, int CO>
@@ -1220,15 +1229,18 @@ LaunchPlan px3_plan(const ConvArgs& a, int out_dtype, bool lif) {
   const Px3Form form = lif ? (lif_resident(a) ? Px3Form::kW32 : Px3Form::kChunks32) : px3_form(a, out_dtype);
   const int co = form == Px3Form::kW32 || form == Px3Form::kChunks32 ? 32 : 64;
   GroupSpread sp;
+  int split = 0;  // tiles up to which four wavefronts walk one
   switch (form) {
-    case Px3Form::kW64: sp = px3w_spread<64>(a); break;
-    case Px3Form::kW32: sp = px3w_spread<32>(a); break;
-    case Px3Form::kStreamed: sp = px3s_spread(a); break;
+    case Px3Form::kW64: sp = px3w_spread<64>(a); split = px3w_split_tiles<64, false>(); break;
+    case Px3Form::kW32:
+      sp = px3w_spread<32>(a);
+      split = lif ? px3w_split_tiles<32, true>() : px3w_split_tiles<32, false>();
+      break;
+    case Px3Form::kStreamed: sp = px3s_spread(a); split = kPx3SplitTiles; break;
     case Px3Form::kChunks32: sp = px3_spread<32>(a); break;
     default: sp = px3_spread<64>(a);
   }
-  const bool split = form != Px3Form::kChunks32 && form != Px3Form::kChunks64 && sp.waves <= kPx3SplitTiles;
-  return {(a.c_out + co - 1) / co * sp.per_group, sp.waves, split ? 4 : 1};
+  return {(a.c_out + co - 1) / co * sp.per_group, sp.waves, sp.waves <= split ? 4 : 1};
 }
 
 int launch_conv_px3(const ConvArgs& a, int in_dtype, int out_dtype, hipStream_t stream) {

@@ -320,6 +320,12 @@ def test_launch_plan_known_shapes():
     assert _plan(32, 256, 14, 14, 384) == (6 * 32, 4, 1)
     assert _plan(128, 256, 14, 14, 192) == (3 * 74, 7, 1)
     assert _plan(16, 256, 14, 14, 384, lif=True) == (12 * 16, 4, 1)
+    # four wavefronts to a tile: up to four tiles a workgroup, two where the
+    # slices are of 32 channels
+    for c_in, lif, upto in ((40, False, 4), (200, False, 4), (100, False, 2), (100, True, 4), (200, True, 0)):
+        seen = {_plan(n, c_in, 16, 16, 64, lif=lif)[1:] for n in range(1, 400)}
+        assert {w for t, w in seen if t <= upto} <= {4} and {w for t, w in seen if t > upto} == {1}
+        assert {t for t, _ in seen} >= {1, 2, 3, 4, 5}
     # other kernels have no such plan
     d = _lib.conv_desc(4, 64, 8, 8, 64, 8, 8, 1, 1, 0, 0, 0)
     with pytest.raises(_lib.UnsupportedError):

@@ -293,15 +293,15 @@ def test_px3_random_shapes(case):
 
 
 # The tiles a workgroup gets on 256 CUs: one tile of one lane; one to four (each
-# walked by four wavefronts, a quarter of the channels each) and five and more
-# (one wavefront); channel groups that end inside a wavefront's quarter; dense
+# walked by four wavefronts, a quarter of the channels each; one and two where
+# 64 < C_in <= 128) and more (one wavefront); channel groups that end inside a wavefront's quarter; dense
 # tiles beside walked ones.  C_in > 128 (streamed), up to 128 and up to 64.
 # Expected: tiles of a pass, wavefronts per tile.
 SPLIT_PLANS = {(1, 132, 1, 1, 20, 1): (1, 4), (2, 160, 5, 13, 4, 1): (1, 4), (64, 129, 16, 16, 64, 1): (1, 4),
                (65, 140, 16, 16, 76, 1): (3, 4), (256, 129, 16, 16, 20, 1): (4, 4), (257, 129, 16, 16, 20, 1): (5, 1),
                (200, 136, 16, 16, 84, 1): (7, 1), (129, 150, 23, 22, 64, 2): (2, 4), (321, 130, 16, 16, 60, 1): (6, 1),
                (1, 100, 1, 1, 20, 1): (1, 4), (2, 128, 5, 13, 36, 1): (1, 4), (64, 65, 16, 16, 64, 1): (2, 4),
-               (200, 100, 15, 14, 76, 2): (3, 4), (100, 66, 16, 16, 76, 1): (5, 1),
+               (200, 100, 15, 14, 76, 2): (3, 1), (70, 100, 15, 14, 76, 1): (4, 1), (100, 66, 16, 16, 76, 1): (5, 1),
                (1, 20, 1, 1, 4, 1): (1, 4), (2, 40, 5, 13, 20, 1): (1, 4), (65, 64, 16, 16, 76, 1): (3, 4),
                (256, 40, 16, 16, 20, 1): (4, 4), (321, 33, 16, 16, 60, 1): (6, 1)}
 SPLIT_CASES = list(SPLIT_PLANS)
