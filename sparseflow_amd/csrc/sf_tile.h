@@ -59,7 +59,9 @@ inline GroupSpread spread_rounds(int64_t tiles, int64_t groups, int64_t even) {
   const int64_t rounds = (groups * ((tiles + kRowsWaves - 1) / kRowsWaves) + cus - 1) / cus;
   const int64_t slots = rounds * cus / groups;  // a group's workgroups in all rounds
   const int64_t waves = rounds <= even ? (tiles + slots - 1) / slots : kRowsWaves;
-  return {(int)waves, (int)((tiles + waves - 1) / waves)};
+  // (A launch holds fewer than 2^32 threads, 1024 to a workgroup: beyond, passes.)
+  const int64_t per_group = (tiles + waves - 1) / waves, most = groups < (1 << 21) ? (1 << 21) / groups : 1;
+  return {(int)waves, (int)(per_group < most ? per_group : most)};
 }
 
 namespace {

@@ -315,6 +315,15 @@ def test_streamed_tiles_take_a_workgroup_per_pass():
     assert _plan(90, 256, 28, 28, 512) == (8 * 79, 16, 1)               # three: full workgroups
 
 
+# Past the threads that a launch holds they make passes too (bitmaps of more
+# frames than their x would fit the card).
+def test_launch_plan_very_many_tiles():
+    for n, c_in, c_out, lif in ((1 << 26, 129, 4, False), (1 << 26, 129, 200, False), (1 << 26, 129, 4, True),
+                                (1 << 26, 100, 4, False)):
+        wg, nt, _ = _plan(n, c_in, 14, 14, c_out, lif=lif)
+        assert 0 < wg <= 1 << 21 and nt == 16
+
+
 def test_launch_plan_known_shapes():
     # six groups of 128 four-row tiles: three tiles each would be 6 x 43 = 258 workgroups
     assert _plan(32, 256, 14, 14, 384) == (6 * 32, 4, 1)
