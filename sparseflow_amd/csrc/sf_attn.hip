@@ -22,8 +22,9 @@
 //
 // Bound by HBM (q, k, v in, y out).  At 256 frames x 12 heads x 196 tokens x
 // 32 (308 MB), inputs new at every call: 64 us = 4.8 TB/s, the card's copy rate
-// (the same inputs again, partly in the last-level cache: 52 us); the form before it, which staged k
-// and v in LDS as f32 and formed KV and the rows on the VALU, took 127 us.
+// (the same inputs again, partly in the last-level cache: 52-57 us); the form
+// before it, which staged k and v in LDS as f32 and formed KV and the rows on
+// the VALU, took 127 us.
 //
 // An item whose KV is not finite everywhere takes its q rows' active elements
 // one by one instead: there an inactive one must not meet a KV row (0 * inf
@@ -257,8 +258,8 @@ int launch_attn_w(AttnArgs a, hipStream_t stream) {
 template <typename T, typename TOut, int D>
 int launch_attn_t(const AttnArgs& a, hipStream_t stream) {
   // A wavefront per item once there are enough items to fill the CUs with
-  // them; a workgroup per item below (2 to 12 items a CU differ by under 5%:
-  // 63.3 against 66.4 us at 12, where the partial sums cost, while a few
+  // them; a workgroup per item below (2 to 12 items a CU differ by under 5%, at
+  // 12 in favour of the first, whose partial sums cost nothing, while a few
   // items on single wavefronts leave most of the GPU idle).
   return a.tb * (int64_t)a.h >= (int64_t)num_cus() * kAttnItemsPerCu ? launch_attn_w<T, TOut, D, 1>(a, stream)
                                                                      : launch_attn_w<T, TOut, D, kAttnWaves>(a, stream);

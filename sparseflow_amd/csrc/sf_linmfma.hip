@@ -907,7 +907,7 @@ double lb_us(const LinShape& s) {  // with the row prescan
 //   37.4;  50000 x 48 -> 192 19.3 -> 16.2;  50000 x 386 -> 384 104 -> 46.6;
 //   701 x 1790 -> 100 112 -> 48.4;  but 50000 x 64 -> 64 13.6 -> 14.5, 100000
 //   x 129 -> 128 35.8 -> 43.6
-//   f32  50176 x 1535 -> 384 479 -> 148;  1000 x 383 -> 384 26.7 -> 15.4;
+//   f32  50176 x 1535 -> 384 480 -> 128;  1000 x 383 -> 384 26.7 -> 15.4;
 //   300 x 50 -> 128 7.6 -> 7.2;  30000 x 161 -> 640 53.7 -> 38.2;  200 x 1001
 //   -> 12 62.2 -> 26.6;  3000 x 99 -> 100 10.9 -> 8.0;  30000 x 200 -> 4 16.6 ->
 //   13.1;  but 65536 x 129 -> 512 65.2 -> 67.4, 100000 x 129 -> 128 37.3 -> 46.7,
